@@ -7,37 +7,51 @@
 // is a weight-streaming problem: every W byte is read once and the MFMA work
 // is negligible.
 //
-// Layout of one launch (grid = N / 16 workgroups of 8 waves):
-//   * a workgroup owns 16 output columns (16 rows of W; gate rows j and up
-//     rows n + j for SwiGLU); wave w takes the K slice [w K / 8, (w + 1) K / 8)
-//     as C = K / 256 chunks of 32;
-//   * x (normalised when fused) is staged once per workgroup in LDS as the
-//     MFMA B operand: 16-byte groups of 8 consecutive k, [k / 8][token slot],
-//     the slot XOR-swizzled by the group index so that the staging writes (a
-//     wave per token, consecutive groups) and the fragment reads (the tokens
-//     of one group) both hit 16 different 16-byte bank groups;
-//   * W fragments (A operand: lane l holds row l % 16, k 8 (l / 16) .. +7) go
-//     from HBM straight into registers: the x loads are issued first (loads
-//     return in order, so staging x waits for x only), then the W fragments
-//     -- all of them, or half when registers are short (SwiGLU's two tiles),
-//     the rest issued once x is staged.  Register use stays low enough for
-//     every workgroup of a launch to be resident, so the whole weight is in
-//     flight at once.  Launches of many rounds of workgroups (lm_head) load
-//     instead in chunk pairs (64 k), each load instruction reading 8 rows x
-//     128 contiguous bytes with 8 consecutive lanes per row, which streams
-//     ~13% faster than 16 rows x 64 bytes; each pair then goes through a 2 KB
-//     wave-private LDS buffer (XOR-swizzled: conflict-free writes of 8 rows
-//     and reads of 16) to become the A fragments.  In a single round of
-//     workgroups the LDS step costs more than the grouping saves;
-//   * one v_mfma_f32_16x16x32_f16 per chunk and tile (tokens >= M are zeros);
-//     the 8 K-slice partials (lane l: rows 4 (l / 16) .. +3, token l % 16)
-//     are summed in LDS and wave 0 applies the epilogue:
+// Layout of one launch (grid = N / columns per workgroup, 8 waves each):
+//   * a workgroup owns TT tiles of R <= 16 output columns (R rows of W each;
+//     SwiGLU: gate rows j and up rows n + j); wave w takes the K slice
+//     [w K / 8, (w + 1) K / 8) as C = K / 256 chunks of 32;
+//   * x is staged in LDS as the MFMA B operand: 16-byte groups of 8
+//     consecutive k, [k / 8][token slot], swizzled (xs_group) so that the
+//     staging writes and the fragment reads spread over the banks.  Without
+//     the norm each wave stages its own K slice of every token (whole 128-byte
+//     lines, no workgroup barrier: nobody else reads it); with the norm each
+//     wave stages whole token rows, whose scale needs the full row;
+//   * every load instruction of W reads 8 rows x 128 contiguous bytes, 8
+//     consecutive lanes per row.  In the MFMA operand pattern (lane l: row
+//     l % 16, 16 rows x 64 bytes) each group of four lanes touches four cache
+//     lines, and the address path, not HBM, sets the rate.  A chunk pair (64
+//     k) then goes through a 2 KB wave-private LDS buffer (XOR-swizzled:
+//     conflict-free writes of 8 rows and reads of 16) to become two A
+//     fragments;
+//   * the loads are non-temporal: no weight byte is used twice in a step, and
+//     whole lines stream 5-10% faster that way (in the 64-byte pattern they
+//     were 10% slower: the second half of a line came from HBM again);
+//   * the x loads go out first (loads return in order, so staging x waits for
+//     x only), then the W loads -- all of them, or as many as the registers
+//     hold beside x, the rest once x is staged -- so that with every workgroup
+//     of a launch resident the whole weight is in flight at once;
+//   * one v_mfma_f32_16x16x32_f16 per chunk and tile.  Up to 8 tokens fill
+//     half of the 16 operand columns, so one x fragment carries chunk c in
+//     columns 0-7 and chunk c + 1 in columns 8-15, and the two chunks
+//     accumulate apart, each using its own half (the other half's sums, and
+//     those of slots past M, are never read);
+//   * the 8 K-slice partials are summed through LDS by one thread per output,
+//     consecutive threads on consecutive columns, which apply the epilogue:
 //       STORE  out[m, n] = acc
-//       ADD    out[m, n] = out[m, n] + acc          (residual stream, in place)
+//       ADD    out[m, n] = out[m, n] + acc          (residual stream, in place;
+//              the old value is loaded with x, off the kernel's tail)
 //       SWIGLU out[m, j] = silu(acc_gate) * acc_up  (W = [2 n, K], gate rows first)
 // The fused RMSNorm computes each token's scale exactly as mce_rmsnorm does
 // (same per-lane chunk order, reduction and rounding), so xn is bit-identical
 // to that op's output.
+//
+// What bounds it (MI355X, 8 tokens, weights from HBM, us per call in graphs of
+// back-to-back calls, previous kernel -> this one): about 2 us of launch, 1 us
+// to the first bytes, the stream at 6.2-7 TB/s and 1 us of tail.  q/k/v (31 MB)
+// 8.7 -> 8.5, o_proj (19 MB) 6.9 -> 5.8, gate/up (101 MB) 20.7 -> 18.9, down
+// (50 MB) 13.9 -> 11.9, lm_head (788 MB) 134.6 -> 121.4; one token: 8.1 ->
+// 7.6, 5.9 -> 5.5, 19.3 -> 17.7, 12.4 -> 11.6, 125.4 -> 113.8.
 #include "mce_common.h"
 
 namespace mce {
@@ -52,216 +66,226 @@ struct DecodeGemmArgs {
   float eps;
 };
 
-// 16-byte group index of k group kg, token slot t in the staged x
+// 16-byte group index of k group kg, token slot t in the staged x.  8 slots:
+// the k groups of a fragment read's two column halves (4 apart) land in
+// different halves of the banks.
 template <int MP>
 __device__ __forceinline__ int xs_group(int kg, int t) {
   if constexpr (MP == 16)
     return kg * 16 + (t ^ (kg & 15));
   else
-    return kg * 8 + (t ^ ((kg >> 1) & 7));
+    return (kg ^ ((kg >> 2) & 1)) * 8 + (t ^ ((kg >> 1) & 7));
 }
 
 __device__ __forceinline__ float silu_mul(float g, float u) {
   return g / (1.0f + __expf(-g)) * u;
 }
+__device__ __forceinline__ u32x4 ld_w(const uint16_t *p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+}
 
-// EPI: 0 store, 1 add, 2 SwiGLU; TT tiles per workgroup (SwiGLU: the gate
-// and up tiles); MP token slots (8 or 16); NORM: fuse RMSNorm; C chunks of 32
-// k per wave; R output columns per tile (16, 12, 10 or 8: lanes of rows >= R
+// A wave's own LDS operations complete in order: only the compiler has to keep
+// the order of its writes and reads.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// EPI: 0 store, 1 add, 2 SwiGLU; TT tiles per workgroup (SwiGLU: half of them
+// gate, half up tiles); MP token slots (8 or 16); NORM: fuse RMSNorm; C chunks
+// of 32 k per wave; R output columns per tile (16, 12, 10 or 8: rows past R
 // re-read row R - 1 and their results are dropped), so that the grid can be
 // sized to a whole number of workgroups per CU.
-// ROWS128: W loads of 8 rows x 128 bytes, fragments rebuilt through LDS.
-template <int EPI, int TT, int MP, bool NORM, int C, int WPE, int R, bool ROWS128>
+// LOOP: the workgroup keeps its staged x and walks a contiguous range of
+// tiles, each chunk pair's registers refilled for the next tile as soon as
+// they are consumed.
+template <int EPI, int TT, int MP, bool NORM, int C, int WPE, int R, bool LOOP>
 __global__ __launch_bounds__(DG_WAVES * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void decode_gemm_kernel(DecodeGemmArgs a) {
   static_assert(R % 2 == 0 && R >= 8 && R <= 16, "tile rows");
   constexpr int K = C * 256;
-  constexpr int VPT = K / 512;      // 16-byte groups of one token row per lane
-  constexpr int NTOK = MP / 8;      // token rows staged per wave
-  // W chunks fetched before x is staged: all of them when the registers of
-  // the W fragments, the x rows and the norm weights fit the occupancy
-  // target together, else half (the rest once x is in LDS)
-  constexpr int REGS = 4 * (TT * C + NTOK * VPT + (NORM ? VPT : 0)) + 24;
-  constexpr int C1 = REGS <= 512 / WPE ? C : (C + 1) / 2;
+  constexpr int XP = MP == 8 ? 2 : 1;  // chunks per x fragment
+  constexpr int VPT = K / 512;         // 16-byte groups of a token slot's x per lane
+  constexpr int NTOK = MP / 8;         // token slots staged per wave
+  // W chunks fetched before x is staged: all that fit beside x (and the norm
+  // weights) at the occupancy target
+  constexpr int NXR = NTOK * VPT + (NORM ? VPT : 0);
+  constexpr int BUDGET = (512 / WPE - 28) / 4 - NXR;
+  constexpr int C1 = BUDGET >= TT * C ? C : (BUDGET / TT) / 2 * 2;
+  constexpr int WXW = TT > 2 ? TT * 256 : 512;  // words per wave: a chunk pair of W, then the partial sums
   __shared__ __attribute__((aligned(16))) uint16_t xs[K / 8 * MP * 8];
-  // ROWS128, per wave: 16 rows x 64 k of W (a chunk pair), row pitch 128
-  // bytes, the 16-byte k group g of row p stored at group g ^ ((p >> 1) & 7)
-  __shared__ __attribute__((aligned(16))) uint32_t wx[ROWS128 ? DG_WAVES : 1][16 * 32];
-  static_assert(K / 8 * MP * 8 * 2 >= DG_WAVES * TT * 4 * 64 * 4, "reduction fits");
+  __shared__ __attribute__((aligned(16))) uint32_t wx[DG_WAVES * WXW];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // first output column of the workgroup (SwiGLU: of its gate / up tile pair)
-  const int col0 = blockIdx.x * (EPI == 2 ? R : R * TT);
+  constexpr int NT = EPI == 2 ? TT / 2 : TT;  // output tiles
   const int r = lane & 15, q = lane >> 4;
+  const int l8 = lane >> 3, k8 = lane & 7;  // row and k group of a 128-byte-row load
 
-  // 1. this wave's token rows of x (and the norm weights)
-  u32x4 xv[NTOK][VPT];
-  u32x4 nw[NORM ? VPT : 1];
+  // 1. x (and the norm weights)
+  u32x4 xv[NTOK][VPT], nw[NORM ? VPT : 1];
 #pragma unroll
-  for (int j = 0; j < NTOK; ++j) {
-    const int m = wave + 8 * j;
-    if (m < a.M) {
-      const uint16_t *xr = a.x + (int64_t)m * a.x_stride;
+  for (int j = 0; j < NTOK; ++j)
+    if constexpr (NORM) {
+      const int m = wave + 8 * j;
+      if (m < a.M) {
+        const uint16_t *xr = a.x + (int64_t)m * a.x_stride;
 #pragma unroll
-      for (int i = 0; i < VPT; ++i)
-        xv[j][i] = *reinterpret_cast<const u32x4 *>(xr + (lane + 64 * i) * 8);
+        for (int i = 0; i < VPT; ++i) xv[j][i] = *reinterpret_cast<const u32x4 *>(xr + (lane + 64 * i) * 8);
+      }
+    } else {
+      const uint16_t *xr = a.x + (int64_t)min(l8 + 8 * j, a.M - 1) * a.x_stride + wave * (K / 8) + 8 * k8;
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) xv[j][i] = *reinterpret_cast<const u32x4 *>(xr + 64 * i);
     }
-  }
   if constexpr (NORM) {
+    if (wave < a.M) {
 #pragma unroll
-    for (int i = 0; i < VPT; ++i)
-      nw[i] = *reinterpret_cast<const u32x4 *>(a.norm_w + (lane + 64 * i) * 8);
-  }
-
-  // 2. first half of the W loads.  ROWS128: load c of a tile reads rows
-  // 8 (c & 1) .. +7 of its 16, lane l taking row 8 (c & 1) + l / 8 at k group
-  // l % 8 of chunk pair c / 2; otherwise load c is chunk c's fragment.
-  static_assert(!ROWS128 || (C % 2 == 0 && C1 % 2 == 0), "chunk pairs");
-  const uint16_t *wp[TT][2];
-#pragma unroll
-  for (int t = 0; t < TT; ++t)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int row = ROWS128 ? (lane >> 3) + 8 * h : r;
-      wp[t][h] = a.w + (int64_t)(col0 + t * (EPI == 2 ? a.N : R) + (row < R ? row : R - 1)) * K +
-                 wave * (K / 8) + 8 * (ROWS128 ? lane & 7 : q);
+      for (int i = 0; i < VPT; ++i) nw[i] = *reinterpret_cast<const u32x4 *>(a.norm_w + (lane + 64 * i) * 8);
     }
-  auto w_addr = [&](int t, int c) {
-    return ROWS128 ? wp[t][c & 1] + 64 * (c >> 1) : wp[t][0] + 32 * c;
-  };
+  }
+  // 2. W: load c of a tile reads rows 8 (c & 1) .. +7 of its 16 at chunk pair
+  // c / 2
   u32x4 wf[TT][C];
+  const uint16_t *wp[TT][2];
+  auto set_tile = [&](int col0) {
 #pragma unroll
-  for (int c = 0; c < C1; ++c)
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-    for (int t = 0; t < TT; ++t) wf[t][c] = *reinterpret_cast<const u32x4 *>(w_addr(t, c));
+      for (int h = 0; h < 2; ++h) {
+        const int trow = EPI == 2 ? (t % NT) * R + (t / NT) * a.N : t * R;
+        wp[t][h] = a.w + (int64_t)(col0 + trow + min(l8 + 8 * h, R - 1)) * K + wave * (K / 8) + 8 * k8;
+      }
+  };
+  auto load_w = [&](int lo, int hi) {
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if (c >= lo && c < hi) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) wf[t][c] = ld_w(wp[t][c & 1] + 64 * (c >> 1));
+      }
+  };
+  const int n_tiles = a.N / (R * NT);
+  int tile = LOOP ? (int)((int64_t)blockIdx.x * n_tiles / gridDim.x) : (int)blockIdx.x;
+  const int tile_end = LOOP ? (int)((int64_t)(blockIdx.x + 1) * n_tiles / gridDim.x) : tile + 1;
+  set_tile(tile * (R * NT));
+  // the output a thread finishes: column oc, token om, tiles ot + OTS p
+  const int oc = tid & 15, om = (tid >> 4) & (MP - 1), ot = tid / (16 * MP);
+  constexpr int OTS = DG_WAVES * 64 / (16 * MP);
+  constexpr int OPT = (NT + OTS - 1) / OTS;
+  uint16_t old[OPT];
+  if constexpr (EPI == 1) {
+#pragma unroll
+    for (int p = 0; p < OPT; ++p) {
+      const int t = min(ot + p * OTS, NT - 1);
+      old[p] = a.out[(int64_t)min(om, a.M - 1) * a.out_stride + tile * (R * NT) + t * R +
+                     min(oc, R - 1)];
+    }
+  }
+  load_w(0, C1);
   // keep these loads ahead of the staging below (the scheduler would
   // otherwise sink most of them past it to save registers)
   __builtin_amdgcn_sched_barrier(0);
 
-  // 3. stage x (normalised) into LDS; slots of tokens >= M hold zeros
+  // 3. stage x (normalised) into LDS; slots past M stay as they are
 #pragma unroll
   for (int j = 0; j < NTOK; ++j) {
-    const int m = wave + 8 * j;
-    if (m < a.M) {
-      float inv = 1.0f;
-      if constexpr (NORM) {
+    if constexpr (NORM) {
+      const int m = wave + 8 * j;
+      if (m < a.M) {
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < VPT; ++i) ss = sumsq8<F16T>(xv[j][i], ss);
-        inv = rms_inv(wave_sum(ss), K, a.eps);
-      }
+        const float inv = rms_inv(wave_sum(ss), K, a.eps);
 #pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        const u32x4 val = NORM ? rms_scale8<F16T>(xv[j][i], nw[NORM ? i : 0], inv) : xv[j][i];
-        *reinterpret_cast<u32x4 *>(&xs[xs_group<MP>(lane + 64 * i, m) * 8]) = val;
+        for (int i = 0; i < VPT; ++i)
+          *reinterpret_cast<u32x4 *>(&xs[xs_group<MP>(lane + 64 * i, m) * 8]) = rms_scale8<F16T>(xv[j][i], nw[i], inv);
       }
     } else {
 #pragma unroll
       for (int i = 0; i < VPT; ++i)
-        *reinterpret_cast<u32x4 *>(&xs[xs_group<MP>(lane + 64 * i, m) * 8]) = u32x4{0, 0, 0, 0};
+        *reinterpret_cast<u32x4 *>(&xs[xs_group<MP>(wave * (C * 4) + 8 * i + k8, l8 + 8 * j) * 8]) = xv[j][i];
     }
   }
+  load_w(C1, C);
+  if constexpr (NORM) lds_barrier();
+  else wave_lds_fence();
 
-  // 4. second half of the W fragments, then the MFMAs
-#pragma unroll
-  for (int c = C1; c < C; ++c)
-#pragma unroll
-    for (int t = 0; t < TT; ++t) wf[t][c] = *reinterpret_cast<const u32x4 *>(w_addr(t, c));
-  lds_barrier();
-  floatx4 acc[TT];
-#pragma unroll
-  for (int t = 0; t < TT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  uint32_t *const wxw = wx[ROWS128 ? wave : 0];
-  // this lane's write slot (row l / 8 + 8 h, k group l % 8) and read slot
-  // (row l % 16, k group 4 hh + l / 16) in the swizzled pair buffer
+  // 4. the MFMAs.  This lane's write slot (row l / 8 + 8 h, k group l % 8) and
+  // read slot (row l % 16, k group 4 hh + l / 16) in the swizzled pair buffer:
+  // row pitch 128 bytes, k group g of row p at group g ^ ((p >> 1) & 7)
+  uint32_t *const wxw = wx + wave * WXW;
   auto wslot = [&](int h) {
-    const int p = (lane >> 3) + 8 * h;
-    return p * 32 + 4 * ((lane & 7) ^ ((p >> 1) & 7));
+    const int p = l8 + 8 * h;
+    return p * 32 + 4 * (k8 ^ ((p >> 1) & 7));
   };
   auto rslot = [&](int hh) { return r * 32 + 4 * ((4 * hh + q) ^ ((r >> 1) & 7)); };
+  for (;;) {
+    floatx4 acc[TT][XP];
 #pragma unroll
-  for (int c = 0; c < C; c += 2) {
-    u32x4 xf[2];
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int kg = (wave * C + c + hh) * 4 + q;
-      xf[hh] = *reinterpret_cast<const u32x4 *>(&xs[xs_group<MP>(kg, r & (MP - 1)) * 8]);
-      if constexpr (MP == 8) xf[hh] = r < 8 ? xf[hh] : u32x4{0, 0, 0, 0};
-    }
+      for (int p = 0; p < XP; ++p) acc[t][p] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (LOOP) set_tile(min(tile + 1, tile_end - 1) * (R * NT));
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      if constexpr (!ROWS128) {
+    for (int c = 0; c < C; c += 2) {
+      u32x4 xg[2];
+#pragma unroll
+      for (int hh = 0; hh < 2 / XP; ++hh) {
+        const int kg = (wave * C + c + hh + (MP == 8 ? r >> 3 : 0)) * 4 + q;
+        xg[hh] = *reinterpret_cast<const u32x4 *>(&xs[xs_group<MP>(kg, r & (MP - 1)) * 8]);
+      }
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        u32x4 f[2];
+        *reinterpret_cast<u32x4 *>(wxw + wslot(0)) = wf[t][c];
+        *reinterpret_cast<u32x4 *>(wxw + wslot(1)) = wf[t][c + 1];
+        wave_lds_fence();
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) f[hh] = *reinterpret_cast<const u32x4 *>(wxw + rslot(hh));
+        wave_lds_fence();
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, wf[t][c + hh]),
-                                                          __builtin_bit_cast(half8, xf[hh]), acc[t],
-                                                          0, 0, 0);
-        continue;
+          acc[t][XP == 2 ? hh : 0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(half8, f[hh]), __builtin_bit_cast(half8, xg[XP == 2 ? 0 : hh]),
+              acc[t][XP == 2 ? hh : 0], 0, 0, 0);
       }
-      // the wave's own LDS operations complete in order: only the compiler
-      // has to keep the writes before the reads (and the next pair's writes
-      // after them)
-      *reinterpret_cast<u32x4 *>(wxw + wslot(0)) = wf[t][c];
-      *reinterpret_cast<u32x4 *>(wxw + wslot(1)) = wf[t][c + 1];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-      u32x4 f[2];
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) f[hh] = *reinterpret_cast<const u32x4 *>(wxw + rslot(hh));
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, f[hh]),
-                                                        __builtin_bit_cast(half8, xf[hh]), acc[t],
-                                                        0, 0, 0);
+      if constexpr (LOOP) load_w(c, c + 2);
     }
-  }
-
-  // 5. sum the K slices: red[wave][tile][component][lane]
-  lds_barrier();  // every wave is done reading xs
-  float *const red = reinterpret_cast<float *>(xs);
+    // 5. partial sums of this wave's K slice, in its own part of wx: component i
+    // of lane l at 64 i + (l ^ 4 i)
+    float *const red = reinterpret_cast<float *>(wxw);
 #pragma unroll
-  for (int t = 0; t < TT; ++t)
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[((wave * TT + t) * 4 + i) * 64 + lane] = acc[t][i];
-  lds_barrier();
-  if (wave != 0 || r >= a.M) return;
-  float v[TT][4];
-#pragma unroll
-  for (int t = 0; t < TT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 4; ++i)
+        red[(t * 4 + i) * 64 + (lane ^ (4 * i))] = XP == 2 ? (r < 8 ? acc[t][0][i] : acc[t][XP - 1][i]) : acc[t][0][i];
+    lds_barrier();
+    const int ri = oc & 3, rl = (16 * (oc >> 2) + om) ^ (4 * ri);
+    auto total = [&](int t) {
       float s = 0.f;
 #pragma unroll
-      for (int sl = 0; sl < DG_WAVES; ++sl) s += red[((sl * TT + t) * 4 + i) * 64 + lane];
-      v[t][i] = s;
-    }
-  // lane holds rows 4 q .. +3 of each tile for token r: output columns
-  // col0 (+ t R) + 4 q .. +3, written as column pairs (rows < R only)
-  if (4 * q >= R) return;
-  constexpr int NOUT = EPI == 2 ? 1 : TT;
-#pragma unroll
-  for (int t = 0; t < NOUT; ++t) {
-    uint32_t *op = reinterpret_cast<uint32_t *>(a.out + (int64_t)r * a.out_stride + col0 + t * R +
-                                                4 * q);
-    float o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = EPI == 2 ? silu_mul(v[0][i], v[TT - 1][i]) : v[t][i];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (4 * q + 2 * h >= R) break;
-      float lo = o[2 * h], hi = o[2 * h + 1];
-      if constexpr (EPI == 1) {
-        const uint32_t old = op[h];
-        lo += F16T::lo(old);
-        hi += F16T::hi(old);
+      for (int sl = 0; sl < DG_WAVES; ++sl) {
+        const float *p = reinterpret_cast<const float *>(wx + sl * WXW) + (t * 4 + ri) * 64;
+        s += p[rl];
+        if constexpr (XP == 2) s += p[rl ^ 8];
       }
-      op[h] = pack2<F16T>(lo, hi);
+      return s;
+    };
+#pragma unroll
+    for (int p = 0; p < OPT; ++p) {
+      const int t = ot + p * OTS;
+      if (t < NT && oc < R && om < a.M) {
+        float o;
+        if constexpr (EPI == 2) o = silu_mul(total(t), total(t + NT));
+        else o = total(t);
+        if constexpr (EPI == 1) o += F16T::lo(old[p]);
+        a.out[(int64_t)om * a.out_stride + tile * (R * NT) + t * R + oc] = F16T::from_float(o);
+      }
     }
+    if (!LOOP || ++tile >= tile_end) return;
+    lds_barrier();  // the sums are read before the next tile's W goes through wx
   }
 }
 
@@ -270,11 +294,15 @@ void launch_dg(const DecodeGemmArgs &a, hipStream_t st) {
   // registers of the W fragments decide how many waves fit per SIMD; every
   // workgroup of a launch should be resident at once
   constexpr int WPE = TT * C <= 24 && MP == 8 ? 4 : 2;
-  const int grid = a.N / (EPI == 2 ? R : R * TT);
-  // many rounds of workgroups (lm_head: 8016 over 256 CUs): 128-byte row loads
-  if constexpr (EPI == 0 && TT == 1 && R == 16) {
+  const int grid = a.N / (EPI == 2 ? R * TT / 2 : R * TT);
+  // Many rounds of workgroups (lm_head: 8016 over 256 CUs).  With 16 token
+  // slots staging x (and its norm) costs a workgroup as much as streaming its
+  // tile: one workgroup per CU keeps x and walks its tiles, 199 -> 129 us at 16
+  // tokens.  With 8 slots the dispatcher's turnover of two workgroups per CU
+  // overlaps the staging and is the faster form (121 against 124-128 us).
+  if constexpr (EPI == 0 && TT == 1 && R == 16 && MP == 16) {
     if (grid >= 8 * cu_count()) {
-      decode_gemm_kernel<EPI, TT, MP, NORM, C, WPE, R, true><<<grid, DG_WAVES * 64, 0, st>>>(a);
+      decode_gemm_kernel<EPI, TT, MP, NORM, C, WPE, R, true><<<cu_count(), DG_WAVES * 64, 0, st>>>(a);
       return;
     }
   }
