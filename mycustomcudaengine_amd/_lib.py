@@ -76,6 +76,13 @@ SIGNATURES = {
                                    _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
 }
 
+# entry points of csrc/mce_internal.h (this package's own, not in the public ABI)
+INTERNAL_SIGNATURES = {
+    "mce_prefill_attention_strided": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int,
+                                               _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64,
+                                               _c_f, _vp]),
+}
+
 _lib = None
 _lock = threading.Lock()
 
@@ -119,7 +126,7 @@ def load() -> ctypes.CDLL:
                 f"{LIB_PATH} is not built; run `python -m mycustomcudaengine_amd.build` "
                 "(no CPU fallback exists for these ops)")
         lib = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_LOCAL)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in (*SIGNATURES.items(), *INTERNAL_SIGNATURES.items()):
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args

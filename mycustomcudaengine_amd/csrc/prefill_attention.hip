@@ -51,6 +51,7 @@
 // ranges, each leaving an unnormalised partial state that
 // prefill_merge_kernel combines by log-sum-exp.
 #include "mce_common.h"
+#include "mce_internal.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -125,6 +126,10 @@ struct PrefillArgs {
   const uint16_t *q, *k, *v;
   uint16_t *out;
   int B, S, Hq, Hkv, G;  // S: query rows (positions) per sequence
+  // elements between consecutive positions and between sequences of q and of
+  // k / v (head rows of 128 are contiguous; paged mode: kv_row only, of the pool)
+  int q_row, kv_row;
+  int64_t q_seq, kv_seq;
   int n_items;
   float scale_log2;
   // paged mode: K / V rows from the page pool [num_blocks, bs, Hkv, 128]
@@ -247,12 +252,13 @@ void prefill_causal_kernel(PrefillArgs a) {
   char *const ks_h = Ks + kh * 2 * TILE;  // this stream's K tiles (2 buffers)
   char *const vs_h = Vs + kh * 2 * TILE;
 
-  const int64_t q_row_stride = (int64_t)a.Hq * PF_HD;
+  const int64_t out_row = (int64_t)a.Hq * PF_HD;
   // this sequence's queries (rows of Hq heads, 256 bytes each; < 2^31 bytes)
-  const i32x4 qrsrc = buffer_rsrc(a.q + (int64_t)b * S * q_row_stride, S * a.Hq * PF_HD * 2);
-  const int kv_row = a.Hkv * PF_HD;  // elements between consecutive keys
-  const uint16_t *kbase = PAGED ? a.k + (int64_t)g * PF_HD : a.k + ((int64_t)b * S * a.Hkv + g) * PF_HD;
-  const uint16_t *vbase = PAGED ? a.v + (int64_t)g * PF_HD : a.v + ((int64_t)b * S * a.Hkv + g) * PF_HD;
+  const uint16_t *const qbase = a.q + b * a.q_seq;
+  const i32x4 qrsrc = buffer_rsrc(qbase, ((S - 1) * a.q_row + a.Hq * PF_HD) * 2);
+  const int kv_row = a.kv_row;  // elements between consecutive keys
+  const uint16_t *kbase = a.k + (PAGED ? 0 : b * a.kv_seq) + (int64_t)g * PF_HD;
+  const uint16_t *vbase = a.v + (PAGED ? 0 : b * a.kv_seq) + (int64_t)g * PF_HD;
   if constexpr (PAGED) {
     // byte offset in the pool of each of the sequence's pages (block ids
     // clamped into the pool), before any K / V load
@@ -278,10 +284,10 @@ void prefill_causal_kernel(PrefillArgs a) {
   // publishes the tile.
   // Unconditional buffer loads: the hardware range check of the descriptor
   // returns zeros for keys at or past the sequence end (the descriptor spans
-  // this (batch, kv head)'s rows up to key S).
+  // this (batch, kv head)'s rows up to the last byte of key S - 1).
   // (paged: the descriptor spans the whole pool; keys past the sequence end
   // are clamped to its last key, which the causal mask hides)
-  const int kv_bytes = PAGED ? (int)(a.cache_bytes - g * PF_HD * 2) : (S * kv_row - g * PF_HD) * 2;
+  const int kv_bytes = PAGED ? (int)(a.cache_bytes - g * PF_HD * 2) : ((S - 1) * kv_row + PF_HD) * 2;
   const i32x4 krsrc = buffer_rsrc(kbase, kv_bytes), vrsrc = buffer_rsrc(vbase, kv_bytes);
   const int la = lane >> 4, lp = lane & 15;
   const int ck = lp ^ la, cv = lp ^ (4 * la);  // chunk this lane fetches (K / V)
@@ -299,6 +305,12 @@ void prefill_causal_kernel(PrefillArgs a) {
     key = min(key, key_S - 1);
     return bt_lds[key >> a.bs_log2] + (key & bsm) * kv_row * 2;
   };
+  // stream index u of this key stream <-> key tile KSPLIT u + kh; contiguous
+  // mode: its byte offset (wave-uniform, the scalar offset of the buffer loads)
+  // is kept running: k_off is that of the K tile staged next, one tile_step
+  // ahead of the V tile staged next
+  const int tile_step = __builtin_amdgcn_readfirstlane(KSPLIT * BN * kv_row * 2);
+  int k_off = 0;
   // paged mode: the pool offsets of this lane's rows of the next K tile to be
   // staged and of the next V tile.  They are looked up one step ahead, once for
   // K and V of a tile, so that no staging load waits for an LDS read (24 / 8
@@ -315,20 +327,17 @@ void prefill_causal_kernel(PrefillArgs a) {
           rows[hh][j] = page_row((tb + KSPLIT * u + kh) * BN + 32 * hh + 4 * (KP * rb + j) + la);
     }
   };
-  // K tile u and V tile u - 1 are staged: on to the next ones
+  // K tile u is staged (and V tile u - 1): on to the next ones
   auto next_rows = [&](int u) {
-    if constexpr (PAGED) {
+    if constexpr (!PAGED) {
+      k_off += tile_step;
+    } else {
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
         for (int j = 0; j < KP; ++j) rows_v[hh][j] = rows_k[hh][j];
       page_rows(u + 1, rows_k);
     }
-  };
-  // stream index u of this key stream <-> key tile KSPLIT u + kh
-  // (wave-uniform, passed as the scalar offset of the buffer loads)
-  auto tile_off = [&](int u) {
-    return __builtin_amdgcn_readfirstlane((KSPLIT * u + kh) * BN * kv_row * 2);
   };
   const int half_bytes = PF_BN * kv_row * 2;  // between the halves of a tile
   // LDS address (m0) of this wave's first block in K / V buffer 0
@@ -349,7 +358,7 @@ void prefill_causal_kernel(PrefillArgs a) {
         for (int j = 0; j < KP; ++j)
           buffer_load_lds16(krsrc, rows_k[hh][j] + voff_k[j], 0, m0 + hh * PF_TILE + j * PF_BLK);
       } else {
-        const int off = tile_off(u) + hh * half_bytes;
+        const int off = k_off + hh * half_bytes;
 #pragma unroll
         for (int j = 0; j < KP; ++j)
           buffer_load_lds16(krsrc, voff_k[j], off, m0 + hh * PF_TILE + j * PF_BLK);
@@ -365,7 +374,7 @@ void prefill_causal_kernel(PrefillArgs a) {
         for (int j = 0; j < KP; ++j)
           buffer_load_lds16(vrsrc, rows_v[hh][j] + voff_v[j], 0, m0 + hh * PF_TILE + j * PF_BLK);
       } else {
-        const int off = tile_off(u) + hh * half_bytes;
+        const int off = k_off - tile_step + hh * half_bytes;
 #pragma unroll
         for (int j = 0; j < KP; ++j)
           buffer_load_lds16(vrsrc, voff_v[j], off, m0 + hh * PF_TILE + j * PF_BLK);
@@ -455,19 +464,20 @@ void prefill_causal_kernel(PrefillArgs a) {
         const int qr = min(r_item + 4 * bq + la, rows_total - 1);
         const int qp = qr / G;
         const int qh = g * G + (qr - qp * G);
-        buffer_load_lds16(qrsrc, (qp * a.Hq + qh) * PF_HD * 2 + ck * 16, 0,
+        buffer_load_lds16(qrsrc, (qp * a.q_row + qh * PF_HD) * 2 + ck * 16, 0,
                           q_m0 + (bq >> 3) * PF_TILE + (bq & 7) * PF_BLK);
       }
     } else {
       const int qh = g * G + (row - qi * G);
-      const uint16_t *qp = a.q + ((int64_t)b * S + (row_ok ? qi : 0)) * q_row_stride +
+      const uint16_t *qp = qbase + (int64_t)(row_ok ? qi : 0) * a.q_row +
                            (int64_t)(row_ok ? qh : 0) * PF_HD + 8 * hf;
 #pragma unroll
       for (int i = 0; i < 8; ++i) qreg[i] = *reinterpret_cast<const u32x4 *>(qp + 16 * i);
     }
+    k_off = __builtin_amdgcn_readfirstlane(kh * BN * kv_row * 2);
     page_rows(0, rows_k);
     stage_k(0);
-    next_rows(0);  // rows_v: tile 0, rows_k: tile 1
+    next_rows(0);  // V: tile 0, K: tile 1
     stage_k(1);
     stage_v(0);
     next_rows(1);
@@ -842,7 +852,7 @@ void prefill_causal_kernel(PrefillArgs a) {
         // non-temporal: the output is not read again by this kernel
         // (back-to-back cfg3 calls 35.2 -> 34.8 us, S = 1024 -2.5 %)
         __builtin_nontemporal_store(val, reinterpret_cast<u32x4 *>(
-                                             a.out + ((int64_t)b * S + p) * q_row_stride +
+                                             a.out + ((int64_t)b * S + p) * out_row +
                                              (int64_t)hh * PF_HD + dim0 + 8 * ch));
       }
     }
@@ -1013,35 +1023,38 @@ int prefill_launch(int dtype, PrefillArgs &a, void *stream, const char *name) {
 
 }  // namespace
 
-extern "C" int mce_prefill_attention(int dtype, const void *query,
-                                     const void *key, const void *value,
-                                     void *output, int batch, int seq_len,
-                                     int num_heads, int num_kv_heads,
-                                     int head_dim, float scale, void *stream) {
+extern "C" int mce_prefill_attention_strided(int dtype, const void *query, const void *key,
+                                             const void *value, void *output, int batch,
+                                             int seq_len, int num_heads, int num_kv_heads,
+                                             int head_dim, int64_t q_seq_stride,
+                                             int64_t q_row_stride, int64_t kv_seq_stride,
+                                             int64_t kv_row_stride, float scale, void *stream) {
   clear_error();
-  MCE_REQUIRE(dtype == MCE_F16 || dtype == MCE_BF16,
-              "mce_prefill_attention: unknown dtype %d", dtype);
-  MCE_REQUIRE(head_dim == PF_HD,
-              "mce_prefill_attention: head_dim must be 128 (got %d)", head_dim);
-  MCE_REQUIRE(batch >= 0 && seq_len >= 0 && num_heads >= 1 && num_kv_heads >= 1,
-              "mce_prefill_attention: bad shape");
-  MCE_REQUIRE(num_heads % num_kv_heads == 0,
-              "mce_prefill_attention: num_heads %d not a multiple of num_kv_heads %d",
-              num_heads, num_kv_heads);
+  const char *name = "mce_prefill_attention";
+  MCE_REQUIRE(dtype == MCE_F16 || dtype == MCE_BF16, "%s: unknown dtype %d", name, dtype);
+  MCE_REQUIRE(head_dim == PF_HD, "%s: head_dim must be 128 (got %d)", name, head_dim);
+  MCE_REQUIRE(batch >= 0 && seq_len >= 0 && num_heads >= 1 && num_kv_heads >= 1, "%s: bad shape",
+              name);
+  MCE_REQUIRE(num_heads % num_kv_heads == 0, "%s: num_heads %d not a multiple of num_kv_heads %d",
+              name, num_heads, num_kv_heads);
   if (batch == 0 || seq_len == 0) return MCE_OK;
-  MCE_REQUIRE(query && key && value && output, "mce_prefill_attention: null pointer");
-  MCE_REQUIRE(aligned16(query) && aligned16(key) && aligned16(value) &&
-                  aligned16(output),
-              "mce_prefill_attention: tensors must be 16-byte aligned");
+  MCE_REQUIRE(query && key && value && output, "%s: null pointer", name);
+  MCE_REQUIRE(aligned16(query) && aligned16(key) && aligned16(value) && aligned16(output),
+              "%s: tensors must be 16-byte aligned", name);
+  MCE_REQUIRE(q_row_stride >= (int64_t)num_heads * head_dim && q_row_stride % 8 == 0 &&
+                  kv_row_stride >= (int64_t)num_kv_heads * head_dim && kv_row_stride % 8 == 0 &&
+                  q_seq_stride >= 0 && q_seq_stride % 8 == 0 && kv_seq_stride >= 0 &&
+                  kv_seq_stride % 8 == 0,
+              "%s: bad strides", name);
   const int G = num_heads / num_kv_heads;
-  MCE_REQUIRE((int64_t)seq_len * G < ((int64_t)1 << 30), "mce_prefill_attention: sequence too long");
-  // one sequence's queries are addressed with 32-bit byte offsets
-  MCE_REQUIRE((int64_t)seq_len * num_heads * head_dim * 2 < ((int64_t)1 << 31),
-              "mce_prefill_attention: seq_len * num_heads too large");
-  // K/V tiles are addressed with 32-bit byte offsets within one batch entry
-  // (including the prefetch of up to 6 64-key tiles past the end)
-  MCE_REQUIRE(((int64_t)seq_len + 512) * num_kv_heads * head_dim * 2 < ((int64_t)1 << 31),
-              "mce_prefill_attention: seq_len * num_kv_heads too large");
+  MCE_REQUIRE((int64_t)seq_len * G < ((int64_t)1 << 30), "%s: sequence too long", name);
+  // one sequence's queries are addressed with 32-bit byte offsets, K/V tiles
+  // likewise (including the prefetch of up to 6 64-key tiles past the end)
+  constexpr int64_t LIM = (int64_t)1 << 30;  // elements
+  MCE_REQUIRE(q_row_stride < LIM && q_row_stride * seq_len < LIM, "%s: seq_len * num_heads too large",
+              name);
+  MCE_REQUIRE(kv_row_stride < LIM && kv_row_stride * ((int64_t)seq_len + 512) < LIM,
+              "%s: seq_len * num_kv_heads too large", name);
   PrefillArgs a{};
   a.q = (const uint16_t *)query;
   a.k = (const uint16_t *)key;
@@ -1052,8 +1065,22 @@ extern "C" int mce_prefill_attention(int dtype, const void *query,
   a.Hq = num_heads;
   a.Hkv = num_kv_heads;
   a.G = G;
+  a.q_row = (int)q_row_stride;
+  a.kv_row = (int)kv_row_stride;
+  a.q_seq = q_seq_stride;
+  a.kv_seq = kv_seq_stride;
   a.scale_log2 = scale * 1.4426950408889634f;
-  return prefill_launch<false>(dtype, a, stream, "mce_prefill_attention");
+  return prefill_launch<false>(dtype, a, stream, name);
+}
+
+extern "C" int mce_prefill_attention(int dtype, const void *query, const void *key,
+                                     const void *value, void *output, int batch, int seq_len,
+                                     int num_heads, int num_kv_heads, int head_dim, float scale,
+                                     void *stream) {
+  const int64_t q_row = (int64_t)num_heads * head_dim, kv_row = (int64_t)num_kv_heads * head_dim;
+  return mce_prefill_attention_strided(dtype, query, key, value, output, batch, seq_len, num_heads,
+                                       num_kv_heads, head_dim, q_row * seq_len, q_row,
+                                       kv_row * seq_len, kv_row, scale, stream);
 }
 
 extern "C" size_t mce_prefill_attention_paged_workspace_size(int batch, int seq_len,
@@ -1113,6 +1140,9 @@ extern "C" int mce_prefill_attention_paged(int dtype, const void *query, const v
   a.Hkv = num_kv_heads;
   a.G = G;
   a.scale_log2 = scale * 1.4426950408889634f;
+  a.q_row = num_heads * head_dim;
+  a.kv_row = num_kv_heads * head_dim;
+  a.q_seq = (int64_t)seq_len * a.q_row;
   a.block_tables = block_tables;
   a.context_lens = context_lens;
   a.maxb = max_blocks_per_seq;

@@ -3,7 +3,7 @@
 prefill_step(model, input_ids [B, S], seq_ids, context_lens) -> last-token
 logits [B, vocab].  Per layer: RMSNorm -> fused q/k/v projection -> RoPE in
 place (positions 0..S-1) and the paged KV store of all B*S tokens in ONE launch ->
-causal prefill attention on the contiguous q/k/v -> o_proj + residual ->
+causal prefill attention reading q/k/v as views of the projection -> o_proj + residual ->
 RMSNorm -> fused gate/up -> SwiGLU -> down + residual; then the final
 RMSNorm and lm_head on the last position only (benchmark_engine.py:124-127).
 

@@ -506,6 +506,26 @@ def decode_advance(block_tables: torch.Tensor, positions: torch.Tensor,
                   int(block_size), cap, _stream(dev))
 
 
+def _seq_row_strides(t: torch.Tensor) -> tuple:
+    """Element strides of [B, S, H, D] between sequences and between positions
+    (a dimension of one element gets its contiguous stride)."""
+    b, s, h, d = t.shape
+    row = t.stride(1) if s > 1 else h * d
+    return (t.stride(0) if b > 1 else row * s), row
+
+
+def _head_rows(t: torch.Tensor) -> bool:
+    """Whether prefill_attention reads the view [B, S, H, D] in place: head rows
+    contiguous and next to each other, positions apart by a multiple of 16
+    bytes, 16-byte aligned, and small enough for 32-bit offsets."""
+    if t.is_contiguous():
+        return True
+    b, s, h, d = t.shape
+    seq, row = _seq_row_strides(t)
+    return (t.stride(3) == 1 and (h == 1 or t.stride(2) == d) and row >= h * d and row % 8 == 0 and
+            seq >= 0 and seq % 8 == 0 and row * (s + 512) < 1 << 30 and t.data_ptr() % 16 == 0)
+
+
 def prefill_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                       scale: float) -> torch.Tensor:
     """Causal GQA attention on contiguous Q/K/V (reference: prefill_attention.cu:271-309).
@@ -523,13 +543,28 @@ def prefill_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tenso
            lambda: f"prefill_attention: key shape {tuple(key.shape)} does not match query "
            f"{tuple(query.shape)}")
     hkv = key.size(2)
-    q = query if query.is_contiguous() else query.contiguous()
-    k = key if key.is_contiguous() else key.contiguous()
-    v = value if value.is_contiguous() else value.contiguous()
-    out = torch.empty_like(q)
+    if not (query.is_contiguous() and key.is_contiguous() and value.is_contiguous()):
+        return _prefill_attention_views(dev, code, query, key, value, scale)
+    out = torch.empty_like(query)
     with _on_device(dev):
-        _lib.call("mce_prefill_attention", code, q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                  out.data_ptr(), b, s, hq, hkv, d, float(scale), _stream(dev))
+        _lib.call("mce_prefill_attention", code, query.data_ptr(), key.data_ptr(),
+                  value.data_ptr(), out.data_ptr(), b, s, hq, hkv, d, float(scale), _stream(dev))
+    return out
+
+
+def _prefill_attention_views(dev, code, query, key, value, scale) -> torch.Tensor:
+    """prefill_attention of strided q, k or v: views into a fused projection are
+    read in place, other layouts copied first."""
+    b, s, hq, d = query.shape
+    q = query if _head_rows(query) else query.contiguous()
+    k, v = key, value
+    if not (_head_rows(k) and _head_rows(v) and k.stride() == v.stride()):
+        k, v = key.contiguous(), value.contiguous()
+    out = torch.empty(b, s, hq, d, dtype=query.dtype, device=dev)
+    with _on_device(dev):
+        _lib.call("mce_prefill_attention_strided", code, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                  out.data_ptr(), b, s, hq, key.size(2), d, *_seq_row_strides(q),
+                  *_seq_row_strides(k), float(scale), _stream(dev))
     return out
 
 

@@ -1,0 +1,64 @@
+"""GPU: layouts and sizes at which a kernel takes another path."""
+import pytest
+import torch
+
+import my_cuda_engine_cpp as ops
+
+pytestmark = pytest.mark.gpu
+
+
+def gen(seed):
+    return torch.Generator().manual_seed(seed)
+
+
+# one shape per launch of the prefill kernel: 64-row items, 128-row items on two
+# key streams (with items left over for a second pick), one key stream
+@pytest.mark.parametrize("b,s,dtype", [(1, 1, torch.float16), (2, 77, torch.bfloat16),
+                                       (1, 1800, torch.float16), (1, 2048, torch.bfloat16),
+                                       (5, 700, torch.float16)])
+def test_prefill_reads_projection_views_in_place(dev, b, s, dtype):
+    """q, k and v as views into one fused projection [B, S, (24 + 8 + 8) 128]
+    give the bits of their contiguous copies, with NaN rows behind every
+    sequence (keys past the end read as zeros, not as the next sequence)."""
+    buf = torch.full((b, s + 3, 40 * 128), float("nan"), dtype=dtype)
+    buf[:, :s] = torch.randn(b, s, 40 * 128, generator=gen(b + s)).to(dtype)
+    buf = buf.to(dev)[:, :s]
+    q = buf[:, :, :3072].unflatten(2, (24, 128))
+    k = buf[:, :, 3072:4096].unflatten(2, (8, 128))
+    v = buf[:, :, 4096:].unflatten(2, (8, 128))
+    got = ops.prefill_attention(q, k, v, 128 ** -0.5)
+    want = ops.prefill_attention(q.contiguous(), k.contiguous(), v.contiguous(), 128 ** -0.5)
+    assert got.is_contiguous() and not torch.isnan(got).any()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_prefill_copies_the_layouts_it_cannot_read(dev):
+    """Transposed heads, k and v of different strides, a misaligned view."""
+    g = gen(7)
+    q, k, v = (torch.randn(2, 90, h, 128, generator=g).half().to(dev) for h in (24, 8, 8))
+    want = ops.prefill_attention(q, k, v, 0.1)
+    qt = q.transpose(1, 2).contiguous().transpose(1, 2)
+    kw = torch.zeros(2, 90, 10, 128, dtype=torch.float16, device=dev)
+    kw[:, :, :8] = k
+    vm = torch.zeros(2 * 90 * 8 * 128 + 1, dtype=torch.float16, device=dev)[1:].view(2, 90, 8, 128)
+    vm.copy_(v)
+    assert torch.equal(ops.prefill_attention(qt, kw[:, :, :8], v, 0.1), want)
+    with pytest.raises(RuntimeError, match="aligned"):  # contiguous but misaligned: refused
+        ops.prefill_attention(q, k, vm, 0.1)
+    qm = torch.zeros(2, 90, 3072 + 4, dtype=torch.float16, device=dev)[:, :, 4:].unflatten(2, (24, 128))
+    qm.copy_(q)
+    assert torch.equal(ops.prefill_attention(qm, k, v, 0.1), want)
+
+
+@pytest.mark.parametrize("n,k", [(33360, 2048), (40976, 3072)])
+def test_decode_gemm_walks_uneven_tile_ranges(dev, n, k):
+    """9-16 tokens on a wide weight: one workgroup per CU walks a contiguous
+    range of 16-column tiles, here of unequal counts; |err| <= 2e-3 + 4e-3 |ref|
+    against fp32 (fp16 rounding of the output and fp32 sums)."""
+    from mycustomcudaengine_amd.ops import decode_gemm
+    g = gen(n)
+    x = torch.randn(13, k, generator=g).half()
+    w = (torch.randn(n, k, generator=g) * 0.02).half()
+    out = decode_gemm(x.to(dev), w.to(dev)).float().cpu()
+    ref = x.float() @ w.float().T
+    assert ((out - ref).abs() <= 2e-3 + 4e-3 * ref.abs()).all()
