@@ -140,6 +140,9 @@ def load() -> ctypes.CDLL:
             raise ImportError(
                 "two HIP runtimes are mapped into this process "
                 f"({sorted(runtimes)}); libmce.so must share torch's")
+        from . import _native
+        _native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                      for name in _native.entries()})
         _lib = lib
         return lib
 

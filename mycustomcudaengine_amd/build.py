@@ -1,8 +1,10 @@
-"""Builds libmce.so (the C-ABI kernel library) in-tree with hipcc for gfx950.
+"""Builds libmce.so (the C-ABI kernel library) in-tree with hipcc for gfx950,
+and _native.so (the Python layer's native calls, host C++ against torch's
+headers).
 
-Replaces the reference's nvcc CUDAExtension build (setup.py:22-42).  There is
-no torch dependency at build time: the library exports only the `extern "C"`
-entry points declared in include/mce_abi.h.
+Replaces the reference's nvcc CUDAExtension build (setup.py:22-42).  libmce.so
+has no torch dependency: it exports the `extern "C"` entry points declared in
+include/mce_abi.h and csrc/mce_internal.h.
 
 Usage:  python -m mycustomcudaengine_amd.build [--jobs N]
 """
@@ -25,6 +27,7 @@ REPO_DIR = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libmce.so")
+NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
 SOURCES = [
     "mce_runtime.hip",
     "elementwise.hip",
@@ -62,6 +65,27 @@ def compile_flags() -> list[str]:
     ]
 
 
+def native_cmd(out: str) -> list[str]:
+    """Host compile and link of the CPython extension module."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no host C++ compiler found")
+    return [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-I{os.path.join(REPO_DIR, 'include')}", f"-I{CSRC}",
+            f"-I{sysconfig.get_paths()['include']}",
+            *[a for p in (*include_paths(), os.path.join(rocm, "include")) for a in ("-isystem", p)],
+            os.path.join(CSRC, "py_ops.cpp"), "-o", out,
+            *[f"-L{p}" for p in library_paths()], "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_python"]
+
+
 def _run(cmd: list[str]) -> None:
     res = subprocess.run(cmd, capture_output=True, text=True)
     # hipcc's host pass warns that it does not know the packed-fp32 feature,
@@ -92,6 +116,8 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
         out = os.path.join(BUILD_DIR, src.replace(".hip", ".s"))
         asm_files.append(out)
         cmds.append([cc, *flags, "--cuda-device-only", "-S", os.path.join(CSRC, src), "-o", out])
+    native_tmp = NATIVE_PATH + ".tmp"
+    cmds.append(native_cmd(native_tmp))
     jobs = jobs or min(len(cmds), os.cpu_count() or 1, 8)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         for cmd, fut in zip(cmds, [ex.submit(_run, c) for c in cmds]):
@@ -110,6 +136,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
     tmp = LIB_PATH + ".tmp"
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs])
     os.replace(tmp, LIB_PATH)
+    os.replace(native_tmp, NATIVE_PATH)
     return LIB_PATH
 
 

@@ -14,7 +14,10 @@ reference's pybind module (csrc/bindings.cpp:4-19,22-29):
 
 Each op validates dtype, device, shape and layout on the host and raises
 RuntimeError (the exception type TORCH_CHECK raises in the reference), then
-calls libmce.so on torch's current HIP stream.  Outputs and the decode
+calls libmce.so on torch's current HIP stream.  Each call first goes to its
+native form (_native, csrc/py_ops.cpp), which takes ordinary GPU tensors in the
+layouts the kernels read and answers NotImplemented to everything else; the
+Python below then checks, copies or reports.  Outputs and the decode
 workspace are allocated with torch, so every op can be recorded by
 torch.cuda.graph (hipGraph).  No op synchronises or reads device memory on the
 host.  There is no CPU path: CPU tensors are rejected.
@@ -24,6 +27,12 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+
+try:
+    from . import _native
+except ImportError as e:
+    raise ImportError(f"{_lib.PKG_DIR}/_native.so is not built or does not load ({e}); run "
+                      "`python -m mycustomcudaengine_amd.build`") from e
 
 __all__ = [
     "rmsnorm",
@@ -86,6 +95,9 @@ class _on_device:
 
 def rmsnorm(input: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """Fused RMSNorm over the last dim (reference: csrc/kernels/rmsnorm.cu:110-130)."""
+    out = _native.rmsnorm(input, weight, eps)
+    if out is not NotImplemented:
+        return out
     dev = _on_gpu("rmsnorm", input, weight)
     code = _dtype_code(input, "rmsnorm input")
     _check(weight.dtype == input.dtype, "rmsnorm: weight dtype must match input")
@@ -104,6 +116,9 @@ def rmsnorm(input: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tens
 
 def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     """silu(first half) * second half of the last dim (reference: swiglu.cu:29-52)."""
+    out = _native.swiglu(gate_up)
+    if out is not NotImplemented:
+        return out
     dev = _on_gpu("swiglu", gate_up)
     code = _dtype_code(gate_up, "swiglu gate_up")
     _check(gate_up.dim() >= 1, "swiglu: input must have at least one dim")
@@ -128,6 +143,9 @@ def paged_kv_store(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tens
     key/value: [N, Hkv, D] (any token/head strides, contiguous last dim);
     caches: contiguous [num_blocks, block_size, Hkv, D]; slot_mapping int32 [N].
     """
+    if _native.paged_kv_store(key, value, key_cache, value_cache,
+                              slot_mapping) is not NotImplemented:
+        return
     dev = _on_gpu("paged_kv_store", key, value, key_cache, value_cache, slot_mapping)
     code = _dtype_code(key, "paged_kv_store key")
     for t, n in ((value, "value"), (key_cache, "key_cache"), (value_cache, "value_cache")):
@@ -179,6 +197,10 @@ def paged_attention_decode(query: torch.Tensor, key_cache: torch.Tensor,
     block_tables int32 [B, max_blocks_per_seq]; context_lens int32 [B].
     Returns a new [B, Hq, D] tensor.  Rows with context_len 0 are zeros.
     """
+    out = _native.paged_attention_decode(query, key_cache, value_cache, block_tables,
+                                         context_lens, max_blocks_per_seq, block_size, scale)
+    if out is not NotImplemented:
+        return out
     dev = _on_gpu("paged_attention_decode", query, key_cache, value_cache,
                   block_tables, context_lens)
     code = _dtype_code(query, "paged_attention_decode query")
@@ -223,6 +245,9 @@ def rope_inplace(query: torch.Tensor, key, cos_table: torch.Tensor,
     query [B, S, Hq, D], key [B, S, Hkv, D] or None (any strides with a
     contiguous last dim); cos/sin fp32 [P, D/2]; positions int32 [B, S].
     """
+    if _native.rope_inplace(query, key, cos_table, sin_table,
+                            positions) is not NotImplemented:
+        return
     tensors = [query, cos_table, sin_table, positions] + ([key] if key is not None else [])
     dev = _on_gpu("rope_inplace", *tensors)
     code = _dtype_code(query, "rope_inplace query")
@@ -267,6 +292,9 @@ def rope_kv_store(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     query_out (contiguous [N, Hq, D]) the rotated query is written there and
     query is left as it was.
     """
+    if _native.rope_kv_store(query, key, value, key_cache, value_cache, cos_table, sin_table,
+                             positions, slot_mapping, query_out) is not NotImplemented:
+        return
     dev = _on_gpu("rope_kv_store", query, key, value, key_cache, value_cache, cos_table,
                   sin_table, positions, slot_mapping)
     code = _dtype_code(query, "rope_kv_store query")
@@ -324,6 +352,11 @@ def decode_rope_attention(query: torch.Tensor, key: torch.Tensor, value: torch.T
     query and key are not modified.  Only for table capacities
     (max_blocks_per_seq * block_size) up to PER_SEQ_MAX_TOKENS.
     """
+    out = _native.decode_rope_attention(query, key, value, key_cache, value_cache, cos_table,
+                                        sin_table, positions, slot_mapping, block_tables,
+                                        context_lens, max_blocks_per_seq, scale)
+    if out is not NotImplemented:
+        return out
     dev = _on_gpu("decode_rope_attention", query, key, value, key_cache, value_cache,
                   cos_table, sin_table, positions, slot_mapping, block_tables, context_lens)
     code = _dtype_code(query, "decode_rope_attention query")
@@ -415,6 +448,10 @@ def decode_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor = None,
     the reference runs these projections through torch.matmul
     (engine/models/llama.py:94-174).
     """
+    if epilogue in _EPILOGUES:
+        y = _native.projection(x, None, None, weight, out, _EPILOGUES[epilogue])
+        if y is not NotImplemented:
+            return y
     dev, code, m, n, k, out = _projection("decode_gemm", x, weight, out, epilogue)
     with _on_device(dev):
         _lib.call("mce_decode_gemm", code, x.data_ptr(), weight.data_ptr(), out.data_ptr(),
@@ -429,6 +466,10 @@ def rmsnorm_decode_gemm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
     launch; the normalised rows are bit-identical to rmsnorm()'s and are not
     written out.  K in {2048, 3072, 4096}.  Replaces the RMSNorm + projection
     pairs of engine/models/llama.py:82-108, :147-159 and :169-174."""
+    if epilogue in _EPILOGUES:
+        y = _native.projection(x, norm_weight, eps, weight, out, _EPILOGUES[epilogue])
+        if y is not NotImplemented:
+            return y
     dev, code, m, n, k, out = _projection("rmsnorm_decode_gemm", x, weight, out, epilogue)
     _check(norm_weight.device == x.device and norm_weight.dtype == x.dtype and
            norm_weight.dim() == 1 and norm_weight.numel() == k and norm_weight.is_contiguous(),
@@ -532,6 +573,9 @@ def prefill_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tenso
 
     query [B, S, Hq, D]; key/value [B, S, Hkv, D].  Returns [B, S, Hq, D].
     """
+    out = _native.prefill_attention(query, key, value, scale)
+    if out is not NotImplemented:
+        return out
     dev = _on_gpu("prefill_attention", query, key, value)
     code = _dtype_code(query, "prefill_attention query")
     _check(key.dtype == query.dtype and value.dtype == query.dtype,
@@ -588,6 +632,10 @@ def prefill_attention_paged(query: torch.Tensor, key_cache: torch.Tensor,
     their keys over several workgroups, merged by a second launch that costs a
     few microseconds even when nothing is split; pass False when the prefixes
     are known to be short."""
+    out = _native.prefill_attention_paged(query, key_cache, value_cache, block_tables,
+                                          context_lens, scale, split_keys)
+    if out is not NotImplemented:
+        return out
     dev = _on_gpu("prefill_attention_paged", query, key_cache, value_cache, block_tables,
                   context_lens)
     code = _dtype_code(query, "prefill_attention_paged query")
