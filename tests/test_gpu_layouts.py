@@ -62,3 +62,21 @@ def test_decode_gemm_walks_uneven_tile_ranges(dev, n, k):
     out = decode_gemm(x.to(dev), w.to(dev)).float().cpu()
     ref = x.float() @ w.float().T
     assert ((out - ref).abs() <= 2e-3 + 4e-3 * ref.abs()).all()
+
+
+# rows of fewer than 64 groups of 8 (flat kernel), 64 and more (row kernel: a
+# partial last workgroup, more rows than grid.y holds), and a call of over 192 MB
+# (non-temporal loads)
+@pytest.mark.parametrize("rows,inter,dtype", [(3, 504, torch.float16), (5, 512, torch.bfloat16),
+                                              (7, 2056, torch.float16), (65540, 512, torch.float16),
+                                              (4100, 8192, torch.bfloat16)])
+def test_swiglu_row_kernels(dev, rows, inter, dtype):
+    """silu(g) u against fp64: half an ulp of the output type plus the fp32
+    exponential's error (2^-11 and 2^-8 of the value, doubled for the sum)."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.empty(rows, 2 * inter, dtype=dtype, device=dev).normal_(generator=g)
+    out = ops.swiglu(x)
+    gate, up = (t.double() for t in x.chunk(2, 1))
+    ref = gate * torch.sigmoid(gate) * up
+    tol = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    assert ((out.double() - ref).abs() <= tol * ref.abs() + 1e-7).all()
