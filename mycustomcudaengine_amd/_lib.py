@@ -81,6 +81,10 @@ INTERNAL_SIGNATURES = {
     "mce_prefill_attention_strided": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int,
                                                _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64,
                                                _c_f, _vp]),
+    "mce_prompt_gemm_takes": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
+    "mce_prompt_gemm_workspace_size": (_c_sz, [_c_int, _c_int, _c_int, _c_int]),
+    "mce_prompt_gemm": (_c_int, [_c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_i64, _c_i64,
+                                 _c_int, _vp, _c_f, _vp, _vp, _c_sz, _vp]),
 }
 
 _lib = None

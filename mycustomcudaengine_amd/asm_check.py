@@ -1,6 +1,7 @@
-"""Wait-state checks for the inline-asm loads of the prefill kernel.
+"""Wait-state checks for the inline-asm loads of the kernels that stage through
+LDS (prefill attention, prompt GEMM).
 
-The prefill kernel's direct-to-LDS buffer loads are inline asm, and the
+Their direct-to-LDS buffer loads are inline asm, and the
 compiler's hazard recognizer does not look inside inline asm, so it cannot
 insert the wait states those loads need.  This scans gfx950 assembly for the
 two rules of gfx9-family parts that apply to them:

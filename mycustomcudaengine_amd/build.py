@@ -34,10 +34,11 @@ SOURCES = [
     "decode_attention.hip",
     "prefill_attention.hip",
     "decode_gemm.hip",
+    "prompt_gemm.hip",
     "decode_loop.hip",
 ]
 # sources whose inline-asm buffer loads are scanned for missing wait states
-ASM_CHECKED = ["prefill_attention.hip"]
+ASM_CHECKED = ["prefill_attention.hip", "prompt_gemm.hip"]
 ARCH = "gfx950"
 
 

@@ -18,6 +18,8 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -43,7 +45,10 @@ namespace {
   X(mce_prefill_attention_paged_workspace_size)                                            \
   X(mce_prefill_attention_paged)                                                           \
   X(mce_decode_gemm)                                                                       \
-  X(mce_rmsnorm_decode_gemm)
+  X(mce_rmsnorm_decode_gemm)                                                               \
+  X(mce_prompt_gemm_takes)                                                                 \
+  X(mce_prompt_gemm_workspace_size)                                                        \
+  X(mce_prompt_gemm)
 struct Entries {
 #define X(name) decltype(&::name) name = nullptr;
   MCE_NATIVE_ENTRIES(X)
@@ -451,6 +456,52 @@ PyObject *projection(PyObject *const *a) {
   return a[4];
 }
 
+// x, weight, out (None: a new tensor), epilogue code, norm weight (None), eps:
+// the projection of a prompt; returns out, or the normalised rows with a norm.
+// Declined where autograd or a dispatch mode has to see the library GEMM.
+PyObject *prompt_gemm(PyObject *const *a) {
+  const at::Tensor *x = plain(a[0]), *w = plain(a[1]), *o = a[2] == Py_None ? nullptr : plain(a[2]),
+                   *nw = a[4] == Py_None ? nullptr : plain(a[4]);
+  int64_t epi;
+  float eps = 0.f;
+  if (!x || !w || (a[2] != Py_None && !o) || (a[4] != Py_None && (!nw || !as_float(a[5], &eps))) ||
+      !as_int(a[3], &epi) || x->dim() != 2 || w->dim() != 2 ||
+      c10::impl::TorchDispatchModeTLS::any_modes_set())
+    return declined();
+  if (at::GradMode::is_enabled())
+    for (const at::Tensor *t : {x, w, o, nw})
+      if (t && t->requires_grad()) return declined();
+  const int code = dtype_code(*x);
+  const int64_t m = x->size(0), k = x->size(1);
+  if (code < 0 || w->scalar_type() != x->scalar_type() || w->device() != x->device() ||
+      w->size(1) != k || x->stride(1) != 1 || !w->is_contiguous() ||
+      (epi == MCE_EPI_SWIGLU && w->size(0) % 2 != 0) || (epi == MCE_EPI_ADD && !o))
+    return declined();
+  const int64_t n = epi == MCE_EPI_SWIGLU ? w->size(0) / 2 : w->size(0);
+  if (!fits_int({m, n, k})) return declined();
+  if (o && (o->scalar_type() != x->scalar_type() || o->device() != x->device() || o->dim() != 2 ||
+            o->size(0) != m || o->size(1) != n || o->stride(1) != 1))
+    return declined();
+  if (nw && (nw->scalar_type() != x->scalar_type() || nw->device() != x->device() || nw->dim() != 1 ||
+             nw->numel() != n || !nw->is_contiguous()))
+    return declined();
+  if (!g_lib.mce_prompt_gemm_takes((int)m, (int)n, (int)k, (int)epi)) return declined();
+  const c10::DeviceGuard guard(x->device());
+  at::Tensor out = o ? *o : at::empty({m, n}, x->options());
+  at::Tensor normed;
+  if (nw) normed = at::empty({m, n}, x->options());
+  const size_t ws_bytes = g_lib.mce_prompt_gemm_workspace_size((int)m, (int)n, (int)k, (int)epi);
+  const Workspace ws(ws_bytes, *x);
+  const void *xp = x->data_ptr(), *wp = w->data_ptr(), *np = nw ? nw->data_ptr() : nullptr;
+  void *op = out.data_ptr(), *yp = nw ? normed.data_ptr() : nullptr, *st = stream_of(x->device());
+  const int64_t xs = x->stride(0), os = out.stride(0);
+  const int rc = launch([&] {
+    return g_lib.mce_prompt_gemm(code, xp, wp, op, (int)m, (int)n, (int)k, xs, os, (int)epi, np, eps, yp,
+                                 ws.ptr, ws_bytes, st);
+  });
+  return result(rc, nw ? normed : out);
+}
+
 // C++ exceptions (torch's allocator, a bad device) become Python errors.
 template <PyObject *(*OP)(PyObject *const *), int N>
 PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -524,6 +575,7 @@ PyMethodDef methods[] = {
     OP("prefill_attention", prefill_attention, 4),
     OP("prefill_attention_paged", prefill_attention_paged, 7),
     OP("projection", projection, 6),
+    OP("prompt_gemm", prompt_gemm, 6),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods,
                       nullptr,               nullptr,   nullptr, nullptr};

@@ -3,9 +3,10 @@
 prefill_step(model, input_ids [B, S], seq_ids, context_lens) -> last-token
 logits [B, vocab].  Per layer: RMSNorm -> fused q/k/v projection -> RoPE in
 place (positions 0..S-1) and the paged KV store of all B*S tokens in ONE launch ->
-causal prefill attention reading q/k/v as views of the projection -> o_proj + residual ->
-RMSNorm -> fused gate/up -> SwiGLU -> down + residual; then the final
-RMSNorm and lm_head on the last position only (benchmark_engine.py:124-127).
+causal prefill attention reading q/k/v as views of the projection -> o_proj +
+residual + RMSNorm -> gate/up + SwiGLU -> down + residual + the next layer's
+RMSNorm (projections.py: one or two launches each, or the library GEMM and the
+separate ops, by size); then the final RMSNorm and lm_head on the last position only (benchmark_engine.py:124-127).
 
 Differences from the reference driver, all defects of it (not semantics):
 the reference builds slot_mapping element by element and launches the KV
@@ -34,6 +35,12 @@ import my_cuda_engine_cpp as ops
 from ..ops import prefill_attention_paged, rope_kv_store
 
 
+def _first_norm(model, x: torch.Tensor) -> torch.Tensor:
+    """RMSNorm in front of layer 0 (the later ones come with the residual add)."""
+    return ops.rmsnorm(x, model.weights["model.layers.0.input_layernorm.weight"],
+                       model.config.rms_norm_eps)
+
+
 def prefill_step(model, input_ids: torch.Tensor, seq_ids: List[int],
                  context_lens: torch.Tensor = None, chunk_size: int = None) -> torch.Tensor:
     c = model.config
@@ -47,17 +54,17 @@ def prefill_step(model, input_ids: torch.Tensor, seq_ids: List[int],
     positions = torch.arange(s, dtype=torch.int32, device=dev).repeat(b, 1).contiguous()
     x = model.weights["model.embed_tokens.weight"][input_ids.reshape(-1)]  # [B*S, hidden]
     kv = cache.kv_cache
+    xn = None
     for l in range(c.num_hidden_layers):
-        p = f"model.layers.{l}"
-        xn = ops.rmsnorm(x, model.weights[f"{p}.input_layernorm.weight"], c.rms_norm_eps)
+        if xn is None:
+            xn = _first_norm(model, x)
         q, k, v = model._attention_block_proj(l, xn)
         q4, k4, v4 = q.view(b, s, hq, d), k.view(b, s, hkv, d), v.view(b, s, hkv, d)
         rope_kv_store(q.view(b * s, hq, d), k.view(b * s, hkv, d), v.view(b * s, hkv, d),
                       kv[l, 0], kv[l, 1], model.cos_table, model.sin_table,
                       positions.view(-1), slots)
         attn = ops.prefill_attention(q4, k4, v4, model.scale)  # [B, S, Hq, D]
-        x.addmm_(attn.view(b * s, hq * d), model.weights[f"{p}.self_attn.o_proj.weight"].T)
-        model._mlp(l, x)
+        xn = model._after_attention(l, attn.view(b * s, hq * d), x)
     last = x.view(b, s, -1)[:, -1].contiguous()
     xf = ops.rmsnorm(last, model.weights["model.norm.weight"], c.rms_norm_eps)
     return torch.matmul(xf, model.lm_head.T)
@@ -82,9 +89,10 @@ def _prefill_chunked(model, input_ids: torch.Tensor, seq_ids: List[int],
         positions = torch.arange(c0, c1, dtype=torch.int32, device=dev).repeat(b, 1).contiguous()
         ctx = torch.full((b,), c1, dtype=torch.int32, device=dev)
         x = model.weights["model.embed_tokens.weight"][input_ids[:, c0:c1].reshape(-1)]
+        xn = None
         for l in range(c.num_hidden_layers):
-            p = f"model.layers.{l}"
-            xn = ops.rmsnorm(x, model.weights[f"{p}.input_layernorm.weight"], c.rms_norm_eps)
+            if xn is None:
+                xn = _first_norm(model, x)
             q, k, v = model._attention_block_proj(l, xn)
             rope_kv_store(q.view(b * n, hq, d), k.view(b * n, hkv, d), v.view(b * n, hkv, d),
                           kv[l, 0], kv[l, 1], model.cos_table, model.sin_table,
@@ -95,8 +103,7 @@ def _prefill_chunked(model, input_ids: torch.Tensor, seq_ids: List[int],
             # at 1024 it is 6% faster to 5% slower, at 512 21% slower)
             attn = prefill_attention_paged(q.view(b, n, hq, d), kv[l, 0], kv[l, 1], tables, ctx,
                                            model.scale, split_keys=c0 >= 1536)
-            x.addmm_(attn.view(b * n, hq * d), model.weights[f"{p}.self_attn.o_proj.weight"].T)
-            model._mlp(l, x)
+            xn = model._after_attention(l, attn.view(b * n, hq * d), x)
     last = x.view(b, -1, x.size(-1))[:, -1].contiguous()
     xf = ops.rmsnorm(last, model.weights["model.norm.weight"], c.rms_norm_eps)
     return torch.matmul(xf, model.lm_head.T)
