@@ -215,54 +215,54 @@ __global__ __launch_bounds__(256) void prompt_sum_kernel(PromptGemmArgs a) {
   *op = v;
 }
 
-// out += sum of the K slices' partials, normed = RMSNorm(out): one wave per
-// row, the row in registers, with mce_rmsnorm's chunk order and arithmetic (its
-// bits for the rounded rows).  Takes the place of the sum and the norm's own
-// launch and read.  VPT 16-byte chunks of a row per lane.
-template <class T, int VPT>
-__global__ __launch_bounds__(64) void prompt_sum_norm_kernel(PromptGemmArgs a) {
-  const int lane = threadIdx.x;
+// out += sum of the K slices' partials, normed = RMSNorm(out): a workgroup per
+// row, a thread per 16-byte chunk of it, so that every load of a row is in
+// flight at once (one wave per row with the row in its registers took 12.4 us
+// at 512 x 3072, 5 slices).  The rounded row goes through LDS, from which every
+// wave takes the sum of squares in mce_rmsnorm's chunk order (its bits).  Takes
+// the place of the sum and of the norm's own launch and read.
+constexpr int PG_NORM_MAX = 4096;
+template <class T>
+__global__ __launch_bounds__(PG_NORM_MAX / 8) void prompt_sum_norm_kernel(PromptGemmArgs a) {
+  __shared__ u32x4 row_lds[PG_NORM_MAX / 8];
+  const int tid = threadIdx.x, lane = tid & 63;
   const int64_t row = blockIdx.x;
-  const int nvec = a.N >> 3;
-  const int64_t total = (int64_t)a.M * a.N;
+  const int nvec = a.N >> 3, idx = min(tid, nvec - 1);
+  const int64_t slice = (int64_t)a.M * a.N / 4;
   u32x4 *const xr = reinterpret_cast<u32x4 *>(a.out + row * a.out_stride);
-  const floatx4 *const pr = reinterpret_cast<const floatx4 *>(a.part + row * a.N);
-  u32x4 v[VPT], wv[VPT];
-  floatx4 s[VPT][2];
+  const floatx4 *const pr = reinterpret_cast<const floatx4 *>(a.part + row * a.N) + 2 * idx;
+  u32x4 v = xr[idx];
+  const u32x4 wv = reinterpret_cast<const u32x4 *>(a.norm_w)[idx];
+  floatx4 s0 = pr[0], s1 = pr[1];
+  for (int p = 1; p < a.split; p += 4) {
+    floatx4 t[4][2];
 #pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    const int idx = min(lane + i * 64, nvec - 1);
-    v[i] = xr[idx];
-    wv[i] = reinterpret_cast<const u32x4 *>(a.norm_w)[idx];
-    s[i][0] = pr[2 * idx];
-    s[i][1] = pr[2 * idx + 1];
-  }
-  for (int p = 1; p < a.split; ++p) {
-    const floatx4 *const pp = pr + p * (total / 4);
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      const int idx = min(lane + i * 64, nvec - 1);
-      s[i][0] += pp[2 * idx];
-      s[i][1] += pp[2 * idx + 1];
+    for (int u = 0; u < 4; ++u) {  // slices past the last re-read it
+      const floatx4 *const pp = pr + min(p + u, a.split - 1) * slice;
+      t[u][0] = pp[0];
+      t[u][1] = pp[1];
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (p + u < a.split) {
+        s0 += t[u][0];
+        s1 += t[u][1];
+      }
   }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const floatx4 &t = k < 2 ? s0 : s1;
+    v[k] = pack2<T>(T::lo(v[k]) + t[2 * (k & 1)], T::hi(v[k]) + t[2 * (k & 1) + 1]);
+  }
+  if (tid < nvec) {
+    xr[tid] = v;
+    row_lds[tid] = v;
+  }
+  lds_barrier();
   float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    const bool in = lane + i * 64 < nvec;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const floatx4 &t = s[i][k >> 1];
-      v[i][k] = pack2<T>(T::lo(v[i][k]) + t[2 * (k & 1)], T::hi(v[i][k]) + t[2 * (k & 1) + 1]);
-    }
-    if (in) xr[lane + i * 64] = v[i];
-    ss = sumsq8<T>(in ? v[i] : u32x4{0, 0, 0, 0}, ss);
-  }
+  for (int i = lane; i < nvec; i += 64) ss = sumsq8<T>(row_lds[i], ss);
   const float inv = rms_inv(wave_sum(ss), a.N, a.eps);
-  u32x4 *const yr = reinterpret_cast<u32x4 *>(a.normed + row * a.N);
-#pragma unroll
-  for (int i = 0; i < VPT; ++i)
-    if (lane + i * 64 < nvec) yr[lane + i * 64] = rms_scale8<T>(v[i], wv[i], inv);
+  if (tid < nvec) reinterpret_cast<u32x4 *>(a.normed + row * a.N)[tid] = rms_scale8<T>(v, wv, inv);
 }
 
 }  // namespace mce
@@ -340,13 +340,8 @@ int prompt_gemm_launch(int dtype, PromptGemmArgs &a, const PromptPlan &p, int ep
   else
     launch_tile<T, PG_STORE>(a, p, st);
   const bool norm = a.norm_w != nullptr;
-  if (norm && a.split > 1 && a.N <= 4096) {
-    if (a.N <= 2048)
-      prompt_sum_norm_kernel<T, 4><<<a.M, 64, 0, st>>>(a);
-    else if (a.N <= 3072)
-      prompt_sum_norm_kernel<T, 6><<<a.M, 64, 0, st>>>(a);
-    else
-      prompt_sum_norm_kernel<T, 8><<<a.M, 64, 0, st>>>(a);
+  if (norm && a.split > 1 && a.N <= PG_NORM_MAX) {
+    prompt_sum_norm_kernel<T><<<a.M, (a.N / 8 + 63) / 64 * 64, 0, st>>>(a);
     return check_launch("mce_prompt_gemm");
   }
   if (a.split > 1) {
