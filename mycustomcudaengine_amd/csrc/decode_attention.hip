@@ -21,6 +21,14 @@
 //   the same wave, so every K/V byte is read from HBM exactly once (the
 //   reference launches one warp per query head and reads each KV row G times).
 //   K/V are streamed with non-temporal loads (each byte is used once).
+//   Few sequences (decode_layout) leave each wave of that layout with a
+//   handful of tiles one after the other, so they take one kv head per
+//   workgroup instead: its 8 waves share the tiles of a range, a range lies in
+//   one sequence, and a query head has as many partials as ranges, an eighth of
+//   the tiles.  (Reading 256-byte slices costs less than the serial tiles
+//   there: one sequence of 2000 tokens 14.9 -> 11.3 us with the merge, 8000 20.7
+//   -> 15.2, 32000 39.2 -> 29.7; two of 8000 24.6 -> 20.2; eight of 32768 are 4 %
+//   slower.)
 //   Short contexts (capacity <= PER_SEQ_MAX_TOKENS) skip the split: the grid
 //   is one 8-wave workgroup per (kv head, sequence), the waves share the
 //   tiles of that head and merge in LDS, and the rows are written directly
@@ -80,6 +88,8 @@ constexpr int MIN_TILES_PER_WG = 4;
 // tiles in the split space and a workgroup that takes a boundary gets that
 // many fewer real tiles.
 constexpr int SEG_TILES = 2;
+// Smallest range of the one-kv-head-per-workgroup split (a tile per wave)
+constexpr int FEW_MIN_TILES = DEC_NW;
 // Context capacities up to this many tokens take the per-sequence mode.
 constexpr int PER_SEQ_MAX_TOKENS = 1024;
 
@@ -153,16 +163,55 @@ __device__ int build_tile_prefix(const DecodeArgs &a, int *pre, int *wave_tot, i
   return carry;
 }
 
+// The same for few sequences: every sequence's tiles padded to whole ranges of
+// `len` tiles, len from an equal share of all tiles up (at least
+// FEW_MIN_TILES) until the padded sequences make no more than J ranges: one
+// range too many would be a second round for some CU.
+__device__ int build_few_prefix(const DecodeArgs &a, int *pre, int *ctx_out, int &len) {
+  const int cap = a.maxb << a.bs_log2;
+  int total = 0;
+  for (int b = 0; b < a.B; ++b) total += (clamp_ctx(a.ctx_lens[b], cap) + TILE - 1) / TILE;
+  len = max(FEW_MIN_TILES, (total + a.J - 1) / a.J);
+  // (one sequence makes at most J; the search ends, as J >= 8 B: decode_layout)
+  for (; a.B > 1; len += 1 + len / 32) {
+    int n = 0;
+    for (int b = 0; b < a.B; ++b)
+      n += ((clamp_ctx(a.ctx_lens[b], cap) + TILE - 1) / TILE + len - 1) / len;
+    if (n <= a.J) break;
+  }
+  int sum = 0;
+  for (int b = 0; b < a.B; ++b) {
+    const int c = clamp_ctx(a.ctx_lens[b], cap);
+    if (threadIdx.x == 0) {
+      pre[b] = sum;
+      ctx_out[b] = c;
+    }
+    sum += ((c + TILE - 1) / TILE + len - 1) / len * len;
+  }
+  if (threadIdx.x == 0) pre[a.B] = sum;
+  lds_barrier();
+  return sum;
+}
+
+// The tile space cut into je ranges: equal shares, or (FEW) `len` tiles each.
+template <bool FEW>
+struct Ranges {
+  int NT, je, len;
+};
 __device__ inline int partition_count(int NT, int J) {
   int je = (NT + MIN_TILES_PER_WG - 1) / MIN_TILES_PER_WG;
   return je < 1 ? 1 : (je > J ? J : je);
 }
-__device__ inline int range_start(int j, int NT, int je) {
-  return (int)((int64_t)j * NT / je);
+template <bool FEW>
+__device__ inline int range_start(int j, const Ranges<FEW> &r) {
+  if constexpr (FEW) return j * r.len;
+  return (int)((int64_t)j * r.NT / r.je);
 }
 // workgroup index that owns tile t
-__device__ inline int owner_of(int t, int NT, int je) {
-  return (int)(((int64_t)(t + 1) * je - 1) / NT);
+template <bool FEW>
+__device__ inline int owner_of(int t, const Ranges<FEW> &r) {
+  if constexpr (FEW) return t / r.len;
+  return (int)(((int64_t)(t + 1) * r.je - 1) / r.NT);
 }
 
 __device__ inline u32x4 ld_nt(const uint16_t *p) {
@@ -219,7 +268,9 @@ __device__ inline u32x4 rope_apply(const u32x4 x, const RopeCS &r, int lr) {
 // 8 query heads per kv head spill a few registers at this occupancy.)
 // FUSED: RoPE + KV append of the new token (per-sequence mode only; a.knew
 // set), a separate instantiation so the plain kernels carry none of its state.
-template <class T, int G, int NW, bool FUSED>
+// FEW: the split with one kv head per workgroup (likewise apart: as a run-time
+// branch it cost the whole-page split up to 6 %).
+template <class T, int G, int NW, bool FUSED, bool FEW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4)))
 void paged_decode_kernel(DecodeArgs a) {
   constexpr int NTH = NW * 64;
@@ -247,7 +298,8 @@ void paged_decode_kernel(DecodeArgs a) {
   __shared__ float red_acc[NW][G][HD];
   __shared__ float red_m[NW][G], red_l[NW][G];
 
-  int NT, je, seg0;  // seg0: virtual tiles at the start of each sequence
+  Ranges<FEW> rg{0, 1, 0};
+  int seg0 = 0;      // virtual tiles at the start of each sequence
   int ctx_j = 0;     // per-sequence mode: the context length, kept for the tile loop
   // fused RoPE + KV append (per-sequence mode): the new token's state
   int pos_j = 0;
@@ -260,7 +312,6 @@ void paged_decode_kernel(DecodeArgs a) {
   int64_t phys_f = 0;      // fused mode: physical block and first row of those rows
   int tv_f = 0;
   if (a.per_seq) {
-    seg0 = 0;
     // one workgroup per (head group, sequence j): a one-sequence tile space
     // [0, tiles of j), so the segment loop below runs once with nparts == 1
     // and the rows are written directly (no merge pass).  The sequence's
@@ -317,9 +368,8 @@ void paged_decode_kernel(DecodeArgs a) {
       pre[j + 1] = (ctx_j + TILE - 1) / TILE;
     }
     lds_barrier();
-    NT = pre[j + 1];
-    je = 1;
-    if (NT == 0) {
+    rg.NT = pre[j + 1];
+    if (rg.NT == 0) {
       for (int i = tid; i < G * HD; i += NTH)
         a.out[((int64_t)j * a.Hq + head0) * HD + i] = 0;
       if (FUSED && w == 0) {  // an empty sequence still gets its new k / v
@@ -332,10 +382,13 @@ void paged_decode_kernel(DecodeArgs a) {
       }
       return;
     }
+  } else if constexpr (FEW) {
+    rg.NT = build_few_prefix(a, pre, ctx_lds, rg.len);
+    rg.je = rg.NT / rg.len;
   } else {
     seg0 = SEG_TILES;
-    NT = build_tile_prefix<NW>(a, pre, wave_tot, ctx_lds);
-    je = partition_count(NT, a.J);
+    rg.NT = build_tile_prefix<NW>(a, pre, wave_tot, ctx_lds);
+    rg.je = partition_count(rg.NT, a.J);
   }
   if (!a.per_seq && j == 0) {
     // rows of empty sequences are zeros; workgroup 0 of each head group
@@ -349,16 +402,16 @@ void paged_decode_kernel(DecodeArgs a) {
       for (int b = tid; b < a.B; b += NTH) {
         int first = 0, n = 0;
         if (pre[b + 1] != pre[b]) {
-          const int jf = owner_of(pre[b] + seg0, NT, je);
+          const int jf = owner_of(pre[b] + seg0, rg);
           first = jf + b;
-          n = owner_of(pre[b + 1] - 1, NT, je) - jf + 1;
+          n = owner_of(pre[b + 1] - 1, rg) - jf + 1;
         }
         *reinterpret_cast<int2 *>(a.ws_meta + 2 * b) = int2{first, n};
       }
   }
-  if (!a.per_seq && j >= je) return;
-  const int t_lo = a.per_seq ? 0 : range_start(j, NT, je);
-  const int t_hi = a.per_seq ? NT : range_start(j + 1, NT, je);
+  if (!a.per_seq && j >= rg.je) return;
+  const int t_lo = a.per_seq ? 0 : range_start(j, rg);
+  const int t_hi = a.per_seq ? rg.NT : range_start(j + 1, rg);
   if (t_lo >= t_hi) return;
 
   // first sequence whose tiles reach past t_lo
@@ -384,8 +437,8 @@ void paged_decode_kernel(DecodeArgs a) {
     const int seg_hi = min(t_hi, pre[b + 1]) - r0;
     const int tok_lo = seg_lo * TILE;
     const int tok_end = min(seg_hi * TILE, ctx);
-    const int j_first = owner_of(r0, NT, je);
-    const int nparts = owner_of(pre[b + 1] - 1, NT, je) - j_first + 1;
+    const int j_first = owner_of(r0, rg);
+    const int nparts = owner_of(pre[b + 1] - 1, rg) - j_first + 1;
 
     // This lane's slice of each query head: dims 8 lr .. 8 lr + 7 as packed
     // 16-bit pairs -- the same dims the lane loads from every K and V row.
@@ -829,15 +882,23 @@ __global__ __launch_bounds__(HD) void paged_decode_merge_kernel(DecodeArgs a) {
 }
 
 struct DecodeLayout {
-  int J, S, hpg, wph, groups;
+  int J, S, hpg, wph, groups, few;
   size_t ml_off, acc_off, meta_off, total;
 };
 
 // S = J + B part slots per query head (compact layout: piece of sequence b in
 // workgroup j at slot j + b), then two ints per sequence (first slot, parts).
-static DecodeLayout decode_layout(int batch, int num_heads, int num_kv_heads) {
+// capacity: tokens a block table holds.
+static DecodeLayout decode_layout(int batch, int num_heads, int num_kv_heads, int64_t capacity) {
   DecodeLayout L{};
-  L.hpg = num_kv_heads < DEC_NW ? num_kv_heads : DEC_NW;
+  // One kv head per workgroup: up to 4 sequences with at least 8 ranges each (8
+  // kv heads: 32 ranges; 4 x 2000-4000 of 32 kv heads, 8 ranges in all, 38.9 ->
+  // 46.8 us), 3 or 4 only while they are short (4 x 6000 25.9 -> 25.7 us, 4 x
+  // 16000 51.5 -> 52.1: the stream is the limit there, and whole pages stream
+  // faster).
+  L.few = batch <= 4 && (int64_t)8 * batch * num_kv_heads <= cu_count() &&
+          (batch <= 2 || batch * capacity <= 49152);
+  L.hpg = L.few ? 1 : (num_kv_heads < DEC_NW ? num_kv_heads : DEC_NW);
   L.wph = DEC_NW / L.hpg;
   L.groups = (num_kv_heads + L.hpg - 1) / L.hpg;
   int J = cu_count() / L.groups;
@@ -864,7 +925,8 @@ extern "C" size_t mce_paged_attention_decode_workspace_size(
     return 0;
   // short contexts run the per-sequence mode, which needs no workspace
   if ((int64_t)max_blocks_per_seq * block_size <= PER_SEQ_MAX_TOKENS) return 0;
-  return decode_layout(batch, num_heads, num_kv_heads).total;
+  return decode_layout(batch, num_heads, num_kv_heads,
+                       (int64_t)max_blocks_per_seq * block_size).total;
 }
 
 namespace {
@@ -917,7 +979,8 @@ int decode_impl(int dtype, const void *query, const void *key_cache, const void 
   MCE_REQUIRE((int64_t)batch * ((int64_t)max_blocks_per_seq * block_size / TILE + 1) <
                   ((int64_t)1 << 30),
               "mce_paged_attention_decode: batch x context too large");
-  const DecodeLayout Lay = decode_layout(batch, num_heads, num_kv_heads);
+  const DecodeLayout Lay = decode_layout(batch, num_heads, num_kv_heads,
+                                         (int64_t)max_blocks_per_seq * block_size);
   const bool per_seq = (int64_t)max_blocks_per_seq * block_size <= PER_SEQ_MAX_TOKENS;
   if (!per_seq && (workspace == nullptr || workspace_bytes < Lay.total ||
                    (reinterpret_cast<uintptr_t>(workspace) & 255) != 0))
@@ -960,6 +1023,7 @@ int decode_impl(int dtype, const void *query, const void *key_cache, const void 
   // final rows, so the launch is one kernel with no partials.  Longer
   // contexts use the balanced split over the concatenated tile space.
   a.per_seq = per_seq ? 1 : 0;
+  const bool few = !per_seq && Lay.few;
   // Per-sequence mode on a grid that leaves CUs idle (few sequences x kv
   // heads): the query heads of a kv head are split over gsplit workgroups
   // (the largest divisor of G that still fits the CUs).  Each reads the same
@@ -983,9 +1047,11 @@ int decode_impl(int dtype, const void *query, const void *key_cache, const void 
 #define MCE_DEC_CASE(TT, GG)                                                   \
   case GG:                                                                     \
     if (a.knew)                                                                \
-      paged_decode_kernel<TT, GG, DEC_NW, true><<<grid, NT_THREADS, 0, st>>>(a); \
+      paged_decode_kernel<TT, GG, DEC_NW, true, false><<<grid, NT_THREADS, 0, st>>>(a); \
+    else if (few)                                                              \
+      paged_decode_kernel<TT, GG, DEC_NW, false, true><<<grid, NT_THREADS, 0, st>>>(a); \
     else                                                                       \
-      paged_decode_kernel<TT, GG, DEC_NW, false><<<grid, NT_THREADS, 0, st>>>(a); \
+      paged_decode_kernel<TT, GG, DEC_NW, false, false><<<grid, NT_THREADS, 0, st>>>(a); \
     break;
 #define MCE_DEC_LAUNCH(TT)                                                     \
   switch (Gw) {                                                                \

@@ -80,3 +80,41 @@ def test_swiglu_row_kernels(dev, rows, inter, dtype):
     ref = gate * torch.sigmoid(gate) * up
     tol = 2.0 ** (-10 if dtype == torch.float16 else -7)
     assert ((out.double() - ref).abs() <= tol * ref.abs() + 1e-7).all()
+
+
+# up to 4 sequences over tables past 1024 tokens take one kv head per workgroup
+# (ranges of whole sequences): contexts at a range's and a tile's edges, an empty
+# sequence, lengths so uneven that the range length has to be searched; the
+# last three stay with the whole-page split (5 sequences, long tables, kv heads)
+@pytest.mark.parametrize("ctx,width,hq,hkv,dtype", [
+    ([1100], 70, 24, 8, torch.float16), ([1], 65, 24, 8, torch.float16),
+    ([128, 129], 66, 24, 8, torch.bfloat16), ([0, 3000], 190, 8, 8, torch.float16),
+    ([17, 5000, 1], 320, 6, 2, torch.float16), ([2048, 33, 0, 1999], 128, 32, 8, torch.bfloat16),
+    ([4000, 100, 4000, 16], 256, 14, 7, torch.float16), ([1500, 7, 900, 16, 2000], 128, 24, 8, torch.float16),
+    ([1, 20000, 5, 300], 1250, 24, 8, torch.float16), ([1100, 3000], 200, 32, 32, torch.float16)])
+def test_decode_of_few_sequences(dev, ctx, width, hq, hkv, dtype):
+    """Against fp64 on the gathered K/V; the unused pool is NaN."""
+    g = gen(sum(ctx) + hq)
+    b, nb = len(ctx), sum(-(-c // 16) for c in ctx) + 3
+    kc, vc = (torch.full((nb, 16, hkv, 128), float("nan"), dtype=dtype) for _ in range(2))
+    tables, perm, off = torch.zeros(b, width, dtype=torch.int32), torch.randperm(nb, generator=g), 0
+    q = torch.randn(b, hq, 128, generator=g).to(dtype)
+    ref = torch.zeros(b, hq, 128, dtype=torch.float64)
+    for i, c in enumerate(ctx):
+        n = -(-c // 16)
+        blocks = perm[off:off + n]
+        off += n
+        tables[i, :n] = blocks.to(torch.int32)
+        k, v = (torch.randn(n * 16, hkv, 128, generator=g).to(dtype) for _ in range(2))
+        k[c:], v[c:] = float("nan"), float("nan")
+        kc[blocks], vc[blocks] = k.view(n, 16, hkv, 128), v.view(n, 16, hkv, 128)
+        if c:
+            kk, vv = (t[:c].double().repeat_interleave(hq // hkv, 1) for t in (k, v))
+            p = torch.softmax(torch.einsum("hd,thd->ht", q[i].double(), kk) * 128 ** -0.5, -1)
+            ref[i] = torch.einsum("ht,thd->hd", p, vv)
+    out = ops.paged_attention_decode(q.to(dev), kc.to(dev), vc.to(dev), tables.to(dev),
+                                     torch.tensor(ctx, dtype=torch.int32, device=dev), width, 16,
+                                     128 ** -0.5).cpu()
+    # P rounds to the element type (2^-11 / 2^-8 relative), |v| <= 5, and so does the output
+    tol = 5 * (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7)
+    assert (out.double() - ref).abs().max().item() <= tol
