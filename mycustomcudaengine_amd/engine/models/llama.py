@@ -29,8 +29,10 @@ batch sizes (at most 8 tokens, fp16, the 3B model's widths) the projections
 run on the decode-sized GEMM kernels: RMSNorm fused in front of the q/k/v and
 gate/up projections, SwiGLU fused behind gate/up, the residual adds fused
 into o_proj / down_proj, the final RMSNorm in front of lm_head -- 4 launches
-per layer besides the attention instead of 7; other shapes use torch.matmul
-(hipBLASLt) with the separate RMSNorm / SwiGLU ops.
+per layer besides the attention instead of 7; 9 to 16 tokens do the same but
+for down_proj.  Other shapes go through projections.py: the prompt GEMM with
+SwiGLU, the residual add and the next RMSNorm fused where it is the faster
+one, torch.matmul (hipBLASLt) with the separate ops otherwise.
 RoPE tables cover max_position_embeddings positions (capped at 131072)
 instead of the reference's fixed 4096 (llama.py:42).
 """
