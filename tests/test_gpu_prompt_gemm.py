@@ -61,6 +61,15 @@ def test_add_norm_equals_add_then_rmsnorm(dev, m, n, k):
     assert torch.equal(a, b) and torch.equal(y, ops.rmsnorm(a, nw, 1e-5))
 
 
+def test_first_call_binds_the_library(dev, monkeypatch):
+    """A process whose first op is a projection takes the same path as a later one."""
+    calls = []
+    load = _lib.load
+    monkeypatch.setattr(_lib, "load", lambda: calls.append(1) or load())
+    linear(rnd(dev, 64, 2048), rnd(dev, 1024, 2048, std=0.02))
+    assert calls
+
+
 def test_takes_and_leaves(dev):
     """Sizes outside its rule, autograd and odd layouts go to the library."""
     lib = _lib.load()
