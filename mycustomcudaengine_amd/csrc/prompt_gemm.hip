@@ -276,22 +276,28 @@ namespace {
 // tokens, up to 256 (in-flight bytes per multiplication, above).  A 256-token
 // tile stays ahead of two of 128 for the unsplit gate/up from M = 257 (M = 300:
 // 47.6 against 59.6 us, 256 against 384 workgroups), for the split projections
-// from M = 385 (M = 300: 37.0 against 33.4; M = 400: 41.3 against 41.8).
+// of long K from M = 385 (M = 300: 37.0 against 33.4; M = 400: 41.3 against
+// 41.8); with short K the partials of its five slices cost more than the tile
+// saves (o_proj with the norm, M = 385: 28.0 against 22.8, 512 32.2 against 26.1).
 struct PromptPlan {
   int bm = 0, bn = 0, mt = 0, nt = 0, split = 1;
 };
 
 // The calls this kernel takes; the library GEMM is the better one elsewhere
-// (3B shapes, library against this kernel): SwiGLU and the residual add up to
-// 512 tokens (M = 700: gate/up 91 against 93 us, M = 2048 down 102 against 111),
-// the plain store up to 128 (M = 200: 20.6 against 21.2), the add of short K
-// (o_proj) up to 256 (M = 300: 18.2 against 19.5), none of 16 tokens and fewer
-// (down 15.5 against 15.9).  Narrower projections were not measured and stay
-// with the library.
+// (3B shapes, library against this kernel): SwiGLU up to 512 tokens (M = 700: 91
+// against 93 us).  The residual add, with the norm behind it on both sides: long
+// K up to 768 (down, M = 512 50.4 against 44.4, 520 52.8 against 51.5, 768 66
+// against 55; 800 64.2 against 64.2, 896 66.8 against 70.2), short K up to 448
+// (o_proj, M = 300 23.5 against 20.5, 384 23.5 against 22.5, 448 24.1 against
+// 23.8; 512 24.7 against 26.1).  The plain store up to 128 (M = 176 19.9 against
+// 21.5, 280 21.3 against 24), and up to 256 the multiples of 32, where the
+// library's time jumps (160 / 192 / 224 / 256: 23.9 / 27.2 / 29.7 / 32.0 against
+// 20.5 / 21.9 / 22.7 / 22.6).  None of 16 tokens and fewer (down 15.5 against
+// 15.9).  Narrower projections were not measured and stay with the library.
 bool prompt_takes(int m, int n, int k, int epilogue) {
   if (m < 17 || n < 1024 || k < 2048 || k % PG_BK != 0 || n % 128 != 0) return false;
-  if (epilogue == MCE_EPI_STORE) return m <= 128;
-  if (epilogue == MCE_EPI_ADD) return m <= (k >= 6144 ? 512 : 256);
+  if (epilogue == MCE_EPI_STORE) return m <= 128 || (m <= 256 && m % 32 == 0);
+  if (epilogue == MCE_EPI_ADD) return m <= (k >= 6144 ? 768 : 448);
   return m <= 512;
 }
 
@@ -302,7 +308,7 @@ PromptPlan prompt_plan(int m, int n, int epilogue, int k) {
     p.bm = p.bn = 64;
   else if (m <= 128)
     p.bm = 128, p.bn = 64;
-  else if (m <= (glu ? 256 : 384))
+  else if (m <= (glu ? 256 : k < 6144 ? 448 : 384))
     p.bm = p.bn = 128;
   else
     p.bm = 256, p.bn = 128;

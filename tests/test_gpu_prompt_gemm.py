@@ -1,4 +1,4 @@
-"""GPU: the prompt GEMM (the engine's projections of 17 to 512 tokens)."""
+"""GPU: the prompt GEMM (the engine's projections of 17 to 768 tokens)."""
 import pytest
 import torch
 
@@ -48,6 +48,26 @@ def test_projections_match_fp64(dev, m, n, k):
     close(a, want, dtype, k)
 
 
+# the residual add's own sizes: short K on the 128-token tile to 448, long K on
+# the 256-token tile past 512; the store's multiples of 32
+@pytest.mark.parametrize("m,n,k,add", [(385, 3072, 3072, True), (448, 3072, 3072, True),
+                                       (513, 3072, 8192, True), (768, 3072, 8192, True),
+                                       (160, 5120, 3072, False), (224, 5120, 3072, False)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_sizes_of_one_epilogue(dev, m, n, k, add, dtype):
+    assert _lib.load().mce_prompt_gemm_takes(m, n, k, 1 if add else 0)
+    x, w = rnd(dev, m, k, dtype=dtype), rnd(dev, n, k, dtype=dtype, std=k ** -0.5)
+    acc = x.double() @ w.double().T
+    if not add:
+        close(linear(x, w), acc, dtype, k)
+        return
+    a, nw = rnd(dev, m, n, dtype=dtype, seed=1), rnd(dev, n, dtype=dtype)
+    want = a.double() + acc
+    y = linear_add_norm(x, w, a, nw, 1e-5)
+    close(a, want, dtype, k)
+    assert torch.equal(y, ops.rmsnorm(a, nw, 1e-5))
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 2048, 2048), (100, 3072, 8192), (256, 3072, 3072),
                                    (500, 3072, 8192), (300, 4096, 6144), (40, 5120, 2048)])
 def test_add_norm_equals_add_then_rmsnorm(dev, m, n, k):
@@ -74,9 +94,10 @@ def test_takes_and_leaves(dev):
     """Sizes outside its rule, autograd and odd layouts go to the library."""
     lib = _lib.load()
     takes = lib.mce_prompt_gemm_takes
+    assert takes(160, 5120, 3072, 0) and takes(448, 3072, 3072, 1) and takes(768, 3072, 8192, 1)
     assert takes(17, 3072, 3072, 0) and takes(512, 3072, 8192, 1) and takes(512, 8192, 3072, 2)
-    for m, n, k, e in ((16, 3072, 3072, 0), (129, 5120, 3072, 0), (257, 3072, 3072, 1),
-                       (513, 3072, 8192, 1), (513, 8192, 3072, 2), (64, 3072, 3080, 0),
+    for m, n, k, e in ((16, 3072, 3072, 0), (129, 5120, 3072, 0), (288, 5120, 3072, 0),
+                       (449, 3072, 3072, 1), (769, 3072, 8192, 1), (513, 8192, 3072, 2), (64, 3072, 3080, 0),
                        (64, 3080, 3072, 0), (64, 512, 3072, 0)):
         assert not takes(m, n, k, e)
         assert lib.mce_prompt_gemm(0, None, None, None, m, n, k, k, n, e, None, 0.0, None, None, 0,
